@@ -403,55 +403,93 @@ __device__ __forceinline__ void adam_step(T (&m)[4], T g_u, T g_v, T omb1, T omb
 
 // ------------------------------------------------------------ row split --
 //
-// Waves per launch the row split aims at: one full round of MI355X's 256
-// CUs.  The two-iteration pass holds 256 registers per lane, one wave per
-// SIMD: 1024 waves (at 1000 x 1000, 119.5 us per launch against 124.0 at
-// 896 and 193.2 at 1088, where a second round starts).  The one-iteration
-// passes get 2048: two waves per SIMD for the float energy and energy +
-// adjoint passes (164 and 179 registers; energy + adjoint 42.3 against
-// 45.4 us at 1024 and 50.5 at 3072; the fused Adam pass 101.4 against
-// 103.8 us).  One geometry serves every one-iteration pass, whatever its
-// dtype and mode, because the finalize and the workspace size are derived
-// from it.  IGM_ENERGY_WAVES and IGM_PAIR_WAVES override them (for tuning
-// sweeps).
+// A pass is one round of equally long waves: the rows of every strip are
+// split into the most row blocks whose thread blocks still run at once on
+// MI355X's 256 CUs.  One block over is a second round as long as the first:
+// a solve of a 757 x 1203 grid took 192 us per two-iteration launch in 258
+// blocks and takes 120 in 252, one of 500 x 500 71 us in 257 blocks and 47
+// in 255; energy + gradient of 1500 x 1500 went from 175 to 146 us (513
+// blocks of two per CU, now 507).  Several rounds are taken only where one row block per strip
+// already needs them (batches), with the split that takes the fewest steps.
+//
+// A wave of R rows takes R steps and `extra` more for its halo, down to one
+// row per wave: on a small grid, where a launch is as long as one wave, the
+// two-iteration pass of a 100 x 100 grid takes 24.4 us per launch of a solve
+// with 1 row per wave, 29.6 with 2 and 39.0 with 4 (the float64 one-iteration
+// pass 41, 52 and 75), though the waves then mostly read each other's rows.
+//
+// Waves that run at once: the two-iteration pass holds 256 registers per
+// lane and 120 KB of LDS per block, one wave per SIMD, 1024 waves.  The float
+// energy and energy + adjoint passes fit two per SIMD, 2048 waves (1000 x
+// 1000, energy + adjoint: 42.3 us against 45.4 at 1024), but the float64 and
+// fused Adam passes one.  One geometry serves every one-iteration pass,
+// because the finalize and the workspace size are derived from it: 2048 as
+// long as its waves have at least kFullRows rows, where the float passes are
+// bound by memory, else 1024, where a second round of short float64 waves
+// costs (256 x 300: 58.7 us against 74.8).
+//
+// IGM_ENERGY_WAVES and IGM_PAIR_WAVES override the number of waves the split
+// aims at, rounded to the nearest (for tuning sweeps).
 constexpr int kTargetWaves = 2048;
 constexpr int kPairTargetWaves = 1024;
-constexpr int kMinRows = 4;  // fewer rows per wave would be mostly halo
+constexpr int kFullRows = 4;
 
-inline int env_waves(const char* name, int dflt) {
+inline int env_waves(const char* name) {
   const char* e = getenv(name);
-  const int r = e ? atoi(e) : dflt;
-  return (r >= 64 && r <= (1 << 20)) ? r : dflt;
+  const int r = e ? atoi(e) : 0;
+  return (r >= 64 && r <= (1 << 20)) ? r : 0;
 }
 inline int target_waves() {
-  static int n = env_waves("IGM_ENERGY_WAVES", kTargetWaves);
+  static int n = env_waves("IGM_ENERGY_WAVES");
   return n;
 }
 inline int pair_target_waves() {
-  static int n = env_waves("IGM_PAIR_WAVES", kPairTargetWaves);
+  static int n = env_waves("IGM_PAIR_WAVES");
   return n;
 }
 
 struct PassGeom {
   int nstrips, nrowblk, blocks;
 };
-// strips of `strip_out` owned columns; the rows of each strip split evenly
-inline PassGeom pass_geom(int nbatch, int Ny, int Nx, int strip_out, int target) {
+// Strips of `strip_out` owned columns, their rows split evenly into nrowblk
+// blocks.  `full`: waves that run at once; `extra`: steps of a wave beyond its
+// rows; `env`: the override, or 0.
+inline PassGeom pass_geom(int nbatch, int Ny, int Nx, int strip_out, int full, int extra, int env) {
   PassGeom g;
   g.nstrips = (Nx + strip_out - 1) / strip_out;
-  const int64_t per = (int64_t)g.nstrips * nbatch;
-  int64_t want = (target + per / 2) / per;
-  const int64_t most = Ny / kMinRows > 1 ? Ny / kMinRows : 1;
-  g.nrowblk = (int)(want < 1 ? 1 : (want > most ? most : want));
-  const int waves = g.nstrips * g.nrowblk;
-  g.blocks = (waves + kWavesPerBlock - 1) / kWavesPerBlock;
+  const auto blocks_of = [&](int64_t n) { return (g.nstrips * n + kWavesPerBlock - 1) / kWavesPerBlock; };
+  const auto rows_in = [&](int64_t n) { return n < 1 ? 1 : (n > Ny ? (int64_t)Ny : n); };
+  int64_t best = 1;
+  if (env) {
+    const int64_t per = (int64_t)g.nstrips * nbatch;
+    best = rows_in((env + per / 2) / per);
+  } else {
+    int64_t best_cost = INT64_MAX;
+    for (int rounds = 1; rounds <= 4; ++rounds) {
+      const int64_t room = (int64_t)rounds * (full / kWavesPerBlock) / nbatch;  // blocks per entry
+      const int64_t n = rows_in(room * kWavesPerBlock / g.nstrips);
+      const int64_t took = (blocks_of(n) * nbatch * kWavesPerBlock + full - 1) / full;
+      const int64_t cost = took * ((Ny + n - 1) / n + extra);
+      if (cost < best_cost) {
+        best_cost = cost;
+        best = n;
+      }
+    }
+  }
+  g.nrowblk = (int)best;
+  g.blocks = (int)blocks_of(best);
   return g;
 }
 // the geometry of the one-iteration passes, and of the two-iteration pass
 inline PassGeom one_pass_geom(int nbatch, int Ny, int Nx) {
-  return pass_geom(nbatch, Ny, Nx, kStripOut, target_waves());
+  const int env = target_waves();
+  const PassGeom g = pass_geom(nbatch, Ny, Nx, kStripOut, kTargetWaves, 1, env);
+  if (env || Ny >= kFullRows * g.nrowblk) return g;
+  return pass_geom(nbatch, Ny, Nx, kStripOut, kTargetWaves / 2, 1, env);
 }
-inline PassGeom pair_pass_geom(int Ny, int Nx) { return pass_geom(1, Ny, Nx, kPairOut, pair_target_waves()); }
+inline PassGeom pair_pass_geom(int Ny, int Nx) {
+  return pass_geom(1, Ny, Nx, kPairOut, kPairTargetWaves, 2, pair_target_waves());
+}
 
 // Fills the physics and vertical-grid fields of the argument block (host).
 template <typename T>
