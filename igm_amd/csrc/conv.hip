@@ -11,12 +11,7 @@
 //  conv_in_kernel       layer 1 (5 -> 32), fp32 VALU (raw inputs such as the
 //                       surface elevation need fp32: bf16 spacing is 16 m at
 //                       2500-3000 m), bias + LeakyReLU, bf16 out.
-//  conv3x3_mfma_kernel  32 -> 32 3x3 layers on v_mfma_f32_16x16x32_bf16:
-//                       forward (bias + LeakyReLU) and dgrad (same kernel,
-//                       flipped/transposed weights, output gated by the
-//                       LeakyReLU derivative of the layer below).  Input
-//                       rows are staged in LDS (pixel stride 80 B: the
-//                       16-B fragment reads of 8 lanes hit distinct banks).
+//  (the 32 -> 32 3x3 layers, forward and data gradient: conv3x3.hip)
 //  head_mfma_kernel     1x1 32 -> 2Nz (<= 32) output layer, fp32 out.
 //  wgrad_mfma_kernel    weight gradient: K = pixels; tiles are transposed
 //                       into LDS as [channel][pixel] (three x-shifted copies
@@ -29,32 +24,12 @@
 //  conv_in_wgrad_kernel layer-1 weight gradient, fp32 VALU.
 //  Adam: per-tensor clip_by_norm + legacy Adam on the fp32 master weights,
 //  then bf16 packing of the MFMA operands.
-#include "common.hpp"
-
-#include <cstdlib>
-#include "../../include/igm_amd.h"
+#include "conv_common.hpp"
 
 namespace igm {
 
-typedef __bf16 bf16;
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-constexpr int kC = 32;        // hidden channels
-constexpr int kCin = 5;       // input fields
 constexpr int kTileW = 64;    // pixels per tile row
-constexpr int kTileH = 4;     // output rows per forward tile (one per wave)
-constexpr int kPxStride = 40; // LDS pixel stride in bf16 (80 B)
 constexpr int kChStride = 72; // LDS channel-row stride in bf16 (144 B) for wgrad
-
-__device__ __forceinline__ float leaky(float x) { return x > 0.f ? x : 0.01f * x; }
-__device__ __forceinline__ float bf2f(bf16 h) { return (float)h; }
-__device__ __forceinline__ bf16 f2bf(float f) { return (bf16)f; }
-
-__device__ __forceinline__ void extent_of(const int32_t* ext, int b, int H, int W, int& ny, int& nx) {
-  ny = ext ? min(ext[2 * b], H) : H;
-  nx = ext ? min(ext[2 * b + 1], W) : W;
-}
 
 // ------------------------------------------------------------ layer 1 --
 // One thread per output pixel.  The 45 inputs of its 3x3 window are loaded
@@ -160,220 +135,6 @@ conv_in_dgrad_kernel(const bf16* __restrict__ dz1, const int32_t* __restrict__ e
   }
 #pragma unroll
   for (int ci = 0; ci < kCin; ++ci) o[ci] = acc[ci];
-}
-
-// ------------------------------------------------ 3x3 MFMA conv (fwd/dgrad) --
-// wt: [9][32 out][32 in] bf16.  MODE 0: out = LeakyReLU(conv + bias).
-// MODE 1 (dgrad): out = conv * (aux > 0 ? 1 : 0.01), aux = activation of the
-// layer below (its sign is the sign of its pre-activation).
-// Block = 4 waves; tile = 4 output rows x 64 pixels; wave w owns row y0 + w.
-// Persistent: logical block k walks tiles [k*per, (k+1)*per) of the tile
-// list ordered with the column-tile index fastest; logical blocks are laid
-// out XCD by XCD (xcd_remap), so each XCD sweeps a band of tile rows and the
-// halo rows and columns of neighbouring tiles meet in its L2.  The 18 weight
-// fragments are loaded once per block.
-template <int MODE>
-__global__ void __launch_bounds__(256)
-conv3x3_mfma_kernel(const bf16* __restrict__ in, const bf16* __restrict__ wt,
-                    const float* __restrict__ bias, const bf16* __restrict__ aux,
-                    const int32_t* __restrict__ ext, int B, int H, int W, int per,
-                    bf16* __restrict__ out) {
-  __shared__ __attribute__((aligned(16))) bf16 tile[kTileH + 2][kTileW + 2][kPxStride];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int nty = (H + kTileH - 1) / kTileH;
-  const int ntx = (W + kTileW - 1) / kTileW;
-  // (32-bit tile indices: the host keeps the activations below 2 GiB, so
-  // there are fewer than 2^25 tiles)
-  const int ntiles = B * ntx * nty;
-  // XCD-contiguous runs of tiles: vertically adjacent tiles (ntx apart in
-  // the x-fastest order) then share one L2 for their halo rows
-  const int t0 = xcd_remap(blockIdx.x, gridDim.x) * per;
-  if (t0 >= ntiles) return;
-  const int t1 = t0 + per < ntiles ? t0 + per : ntiles;
-
-  // weight fragments: A operand (16 out-channels x 32 in-channels per tap)
-  bf16x8 wf[9][2];
-#pragma unroll
-  for (int t = 0; t < 9; ++t)
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb)
-      wf[t][cb] = *reinterpret_cast<const bf16x8*>(wt + ((t * kC + cb * 16 + (lane & 15)) * kC + 8 * (lane >> 4)));
-  float bias_r[2][4];
-  if constexpr (MODE == 0) {
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) bias_r[cb][e] = bias[cb * 16 + 4 * (lane >> 4) + e];
-  }
-
-  // Staging of a tile's input rows y0-1 .. y0+4, pixels x0-1 .. x0+64 (zero
-  // outside the entry's extent): kChunks 16-B chunks, kPerThread per thread,
-  // all loads issued before any is used.  The next tile's loads are issued
-  // before the current tile's MFMAs, so they are in flight during them.
-  constexpr int kChunks = (kTileH + 2) * (kTileW + 2) * 4;
-  constexpr int kPerThread = (kChunks + 255) / 256;
-  uint4 stage[kPerThread];
-  struct Tile {
-    int b, y0, x0, ny, nx;
-    bool valid;
-  };
-  auto tile_of = [&](int ti) {
-    Tile t;
-    t.x0 = (ti % ntx) * kTileW;
-    t.y0 = ((ti / ntx) % nty) * kTileH;
-    t.b = ti / (nty * ntx);
-    extent_of(ext, t.b, H, W, t.ny, t.nx);
-    t.valid = t.y0 < t.ny && t.x0 < t.nx;
-    return t;
-  };
-  // branch-free staging loads of tile ti (all masked when ti >= t1 or the
-  // tile is padding): the destination registers stay fixed across the loop
-  const rsrc_t rin = make_rsrc(in, (uint32_t)((int64_t)B * H * W * kC * 2));
-  auto issue_loads = [&](const Tile& t, bool live) {
-    const int64_t img = (int64_t)t.b * H * W;
-#pragma unroll
-    for (int k = 0; k < kPerThread; ++k) {
-      const int c = tid + 256 * k;
-      const int chunk = c & 3;
-      const int px = (c >> 2) % (kTileW + 2);
-      const int row = (c >> 2) / (kTileW + 2);
-      const int yy = t.y0 - 1 + row, xx = t.x0 - 1 + px;
-      const bool ok = live && t.valid && c < kChunks && yy >= 0 && yy < t.ny && xx >= 0 && xx < t.nx;
-      const uint32_t off = ok ? (uint32_t)(((img + (int64_t)yy * W + xx) * kC + chunk * 8) * 2) : kOOB;
-      const auto v = __builtin_amdgcn_raw_buffer_load_b128(rin, off, 0, 0);
-      stage[k] = uint4{v[0], v[1], v[2], v[3]};
-    }
-  };
-
-  Tile cur = tile_of(t0);
-  issue_loads(cur, true);
-  for (int ti = t0; ti < t1; ++ti) {
-    const int64_t img = (int64_t)cur.b * H * W;
-    const int y = cur.y0 + wave;
-    const int x0 = cur.x0;
-    const int ny = cur.ny, nx = cur.nx;
-    if (!cur.valid) {  // tile outside the valid region: zeros (block-uniform)
-      cur = tile_of(ti + 1 < t1 ? ti + 1 : ti);
-      issue_loads(cur, ti + 1 < t1);
-      if (y < H) {
-        const int x = x0 + lane;
-        if (x < W) {
-          uint4 z = {0, 0, 0, 0};
-          uint4* o = reinterpret_cast<uint4*>(out + ((img + (int64_t)y * W + x) * kC));
-#pragma unroll
-          for (int q = 0; q < 4; ++q) o[q] = z;
-        }
-      }
-      continue;
-    }
-    // (the compute below is reached only through this path, after the wait
-    // for the staged loads, so the compiler places no memory waits in it)
-    // MODE 1: the epilogue's activation signs are loaded here, before the
-    // barrier and so before the next tile's staging loads.  Loads complete
-    // in issue order, so the epilogue's wait for them leaves the staging
-    // loads in flight (issued after them, it would wait for those too).
-    uint2 auxv[4][2];
-    if constexpr (MODE == 1) {
-      const rsrc_t raux = make_rsrc(aux, (uint32_t)((int64_t)B * H * W * kC * 2));
-#pragma unroll
-      for (int pb = 0; pb < 4; ++pb) {
-        const int x = x0 + pb * 16 + (lane & 15);
-        const bool ok = y < H && x < W;
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb) {
-          const int co = cb * 16 + 4 * (lane >> 4);
-          const uint32_t off = ok ? (uint32_t)(((img + (int64_t)y * W + x) * kC + co) * 2) : kOOB;
-          const auto v = __builtin_amdgcn_raw_buffer_load_b64(raux, off, 0, 0);
-          auxv[pb][cb] = uint2{v[0], v[1]};
-        }
-      }
-    }
-    __syncthreads();  // the previous tile's fragment reads are done
-#pragma unroll
-    for (int k = 0; k < kPerThread; ++k) {
-      const int c = tid + 256 * k;
-      if (c < kChunks) {
-        const int chunk = c & 3;
-        const int px = (c >> 2) % (kTileW + 2);
-        const int row = (c >> 2) / (kTileW + 2);
-        *reinterpret_cast<uint4*>(&tile[row][px][chunk * 8]) = stage[k];
-      }
-    }
-    __syncthreads();
-    cur = tile_of(ti + 1 < t1 ? ti + 1 : ti);
-    issue_loads(cur, ti + 1 < t1);
-
-    f32x4 acc[4][2];
-#pragma unroll
-    for (int pb = 0; pb < 4; ++pb)
-#pragma unroll
-      for (int cb = 0; cb < 2; ++cb) acc[pb][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-#pragma unroll
-    for (int pb = 0; pb < 4; ++pb) {
-      bf16x8 bfr[9];
-#pragma unroll
-      for (int t = 0; t < 9; ++t)
-        bfr[t] = *reinterpret_cast<const bf16x8*>(
-            &tile[wave + t / 3][pb * 16 + (lane & 15) + t % 3][8 * (lane >> 4)]);
-#pragma unroll
-      for (int t = 0; t < 9; ++t) {
-        acc[pb][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[t][0], bfr[t], acc[pb][0], 0, 0, 0);
-        acc[pb][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[t][1], bfr[t], acc[pb][1], 0, 0, 0);
-      }
-    }
-
-    if (y < H) {
-#pragma unroll
-      for (int pb = 0; pb < 4; ++pb) {
-        const int x = x0 + pb * 16 + (lane & 15);
-        if (x >= W) continue;
-        const bool valid = (y < ny) && (x < nx);
-        const int64_t po = (img + (int64_t)y * W + x) * kC;
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb) {
-          const int co = cb * 16 + 4 * (lane >> 4);
-          float v[4];
-          if constexpr (MODE == 0) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = leaky(acc[pb][cb][e] + bias_r[cb][e]);
-          } else {
-            const bf16* g = reinterpret_cast<const bf16*>(&auxv[pb][cb]);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = acc[pb][cb][e] * (bf2f(g[e]) > 0.f ? 1.f : 0.01f);
-          }
-          bf16 h[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) h[e] = valid ? f2bf(v[e]) : f2bf(0.f);
-          *reinterpret_cast<uint2*>(out + po + co) = *reinterpret_cast<const uint2*>(h);
-        }
-      }
-    }
-  }
-}
-
-// persistent grid for the 3x3 kernels: enough blocks to fill the chip a few
-// times over, each walking a contiguous run of tiles
-// 512 blocks (2 per CU, each pipelining a run of ~8 tiles): measured at
-// 1000 x 1000, 35.3 us per 32->32 layer against 36.6 / 39.5 / 46.2 us for
-// 1024 / 2048 / 4096 blocks and 48.6 us for 256.  (IGM_CONV_BLOCKS
-// overrides the target block count, for tuning sweeps.)
-inline int64_t conv_target_blocks() {
-  static int64_t n = [] {
-    const char* e = getenv("IGM_CONV_BLOCKS");
-    const long long r = e ? atoll(e) : 512;
-    return (int64_t)((r >= 64 && r <= (1 << 22)) ? r : 512);
-  }();
-  return n;
-}
-
-inline void conv_grid(int B, int H, int W, int* blocks, int* per) {
-  const int64_t nty = (H + kTileH - 1) / kTileH, ntx = (W + kTileW - 1) / kTileW;
-  const int64_t ntiles = (int64_t)B * nty * ntx;
-  const int64_t kTarget = conv_target_blocks();
-  const int64_t p = (ntiles + kTarget - 1) / kTarget;
-  *per = (int)(p < 1 ? 1 : p);
-  *blocks = (int)((ntiles + *per - 1) / *per);
 }
 
 // ------------------------------------------------------- 1x1 head (MFMA) --
@@ -538,10 +299,6 @@ head_bwd_kernel(const float* __restrict__ dY, const bf16* __restrict__ a16,
 // s=0 is the first read, s=2 a dword select, s=1 a 16-bit funnel shift
 // (v_alignbit).  A block loads its next tile into registers before the
 // current tile's MFMAs.  partials: [gridDim.x][TAPS*1024 + 32] fp32.
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
-
 constexpr int kWgRows = 4;  // dZ rows per tile (8 measured slower on c4 batches)
 
 template <int TAPS>
@@ -1020,38 +777,6 @@ int igm_conv_in_fwd(const float* f0, const float* f1, const float* f2, const flo
   hipLaunchKernelGGL(conv_in_kernel, dim3(grid_for(W), H, B), dim3(256), 0, (hipStream_t)stream,
                      f0, f1, f2, f3, f4, fb, fr, fc, extents, H, W, w_hwio, bias,
                      (bf16*)out_bf16);
-  IGM_CHECK_LAUNCH();
-  return 0;
-}
-
-int igm_conv3x3_fwd_bf16(const void* in, const void* wpacked, const float* bias,
-                         const int32_t* extents, int32_t B, int32_t H, int32_t W, void* out,
-                         void* stream) {
-  IGM_CHECK_ARG(in && wpacked && bias && out, "null pointer");
-  IGM_CHECK_ARG(in != out, "in and out must differ");
-  IGM_CHECK_ARG(B >= 1 && H >= 1 && W >= 1 && B <= 65535, "bad sizes");
-  IGM_CHECK_ARG((int64_t)B * H * W * kC * 2 < (int64_t)kOOB, "activations above 2 GiB (32-bit buffer offsets)");
-  int blocks, per;
-  conv_grid(B, H, W, &blocks, &per);
-  hipLaunchKernelGGL(conv3x3_mfma_kernel<0>, dim3(blocks), dim3(256), 0, (hipStream_t)stream,
-                     (const bf16*)in, (const bf16*)wpacked, bias, (const bf16*)nullptr, extents, B, H, W,
-                     per, (bf16*)out);
-  IGM_CHECK_LAUNCH();
-  return 0;
-}
-
-int igm_conv3x3_dgrad_bf16(const void* dz, const void* wpacked_dgrad, const void* act_below,
-                           const int32_t* extents, int32_t B, int32_t H, int32_t W, void* dz_below,
-                           void* stream) {
-  IGM_CHECK_ARG(dz && wpacked_dgrad && act_below && dz_below, "null pointer");
-  IGM_CHECK_ARG(dz != dz_below, "in and out must differ");
-  IGM_CHECK_ARG(B >= 1 && H >= 1 && W >= 1 && B <= 65535, "bad sizes");
-  IGM_CHECK_ARG((int64_t)B * H * W * kC * 2 < (int64_t)kOOB, "activations above 2 GiB (32-bit buffer offsets)");
-  int blocks, per;
-  conv_grid(B, H, W, &blocks, &per);
-  hipLaunchKernelGGL(conv3x3_mfma_kernel<1>, dim3(blocks), dim3(256), 0, (hipStream_t)stream,
-                     (const bf16*)dz, (const bf16*)wpacked_dgrad, (const float*)nullptr,
-                     (const bf16*)act_below, extents, B, H, W, per, (bf16*)dz_below);
   IGM_CHECK_LAUNCH();
   return 0;
 }

@@ -1,0 +1,465 @@
+// The emulator's 32 -> 32 3x3 layers on gfx950 (v_mfma_f32_16x16x32_bf16):
+// forward (bias + LeakyReLU), data gradient, and two forward layers in one
+// launch (emulate/neural_network.py:9-66).
+//
+// A wave owns a strip of 64 pixel columns and walks down its rows with the
+// three input rows of a 3x3 window in registers, loading the next one while
+// it multiplies.  A product takes 16 output channels (A: the weights, one
+// 16-B fragment per lane and tap from LDS) and 16 pixels (B: lane n + 16 g
+// holds channels 8 g .. 8 g + 7 of pixel slot n, the 16 B that NHWC rows hold
+// them in, so activations go from memory to the products without LDS).  The
+// weight rows are taken in the order that leaves a lane with 8 consecutive
+// channels of its pixel: 16-B stores, and the layout of the next layer's
+// operand.  Every output sums taps 0 .. 8 in order from zero and adds the
+// bias last, in all of these kernels: they agree bit for bit.
+//
+// What bounds them: at 1000 x 1000 one layer moves 128 MB in 22.6 us, the
+// rate of a plain copy of such buffers (23 to 25 us; 5.7 TB/s), where the
+// products alone take 7.5 us.  The earlier kernel, which staged tiles of rows
+// in LDS between barriers, took 33 us.  Two layers in one launch move half
+// the bytes and are bound by instruction issue: a product takes 8 of its 16
+// matrix cycles of the SIMD's issue and the other instructions 4 each, about
+// 150 of them per 72 products.  37 to 42 us for both at 1000 x 1000, 8.5 at
+// 100 x 100 (5.1 for one).
+#include "conv_common.hpp"
+
+namespace igm {
+
+constexpr int kStripPx = 64;            // pixels of a wave's row
+constexpr int kPairPx = kStripPx - 2;   // columns a wave of the two-layer kernel owns
+
+// cache policy of a kernel's stores: cached, non-temporal, written through
+constexpr int kStoreCached = 0, kStoreStream = 2, kStoreThrough = 16;
+
+struct ConvGeom {
+  int nstrips, nrowblk, rows, blocks;
+};
+// Strips of `own` columns, their rows in blocks of `rows`: the most blocks
+// that leave one wave per SIMD, 1024 in all (256 x 319: 7.4 us a layer, 8.8
+// with 2048; 1000 x 1000: 24.9 and 25.9), so that every wave of one field
+// takes as long.  In a batch of uneven entries (ext) some waves only write
+// padding; blocks of at most 32 rows keep the others short enough to fill in
+// for them.  The two-layer kernel holds one wave per SIMD, so it keeps to one
+// round instead.  (IGM_CONV_BLOCKS overrides the number of blocks of four
+// waves the split aims at, for tuning sweeps.)
+constexpr int kConvBlocks = 256;
+constexpr int kConvRows = 32;
+inline int64_t conv_target_waves() {
+  static const int64_t n = [] {
+    const char* e = getenv("IGM_CONV_BLOCKS");
+    const long long r = e ? atoll(e) : kConvBlocks;
+    return 4 * (int64_t)((r >= 64 && r <= (1 << 22)) ? r : kConvBlocks);
+  }();
+  return n;
+}
+inline ConvGeom conv_geom(int B, int H, int W, int own, bool ext) {
+  ConvGeom c;
+  c.nstrips = (W + own - 1) / own;
+  const int64_t strips = (int64_t)B * c.nstrips;
+  const int64_t blk = conv_target_waves() / strips < 1 ? 1 : conv_target_waves() / strips;
+  const int64_t rows = (H + blk - 1) / blk;
+  c.rows = (int)(ext && own == kStripPx && rows > kConvRows ? kConvRows : rows);
+  c.nrowblk = (H + c.rows - 1) / c.rows;
+  c.blocks = (int)((strips * c.nrowblk + 3) / 4);
+  return c;
+}
+
+struct ConvArgs {
+  const bf16* in;
+  const bf16* wt[2];
+  const float* bias[2];
+  const bf16* aux;
+  bf16* out;
+  const int32_t* ext;
+  int B, H, W;
+  ConvGeom g;
+};
+
+// This wave's part of the image.
+struct ConvTile {
+  int lane, n, g;  // pixel slot n of 16, channel group g of 4 (8 channels each)
+  int x0, y0, y1;  // first column, rows
+  int ny, nx;
+  uint32_t bytes, rowbytes, img;
+  bool live;
+};
+__device__ __forceinline__ ConvTile conv_tile(const ConvArgs& a, int own) {
+  ConvTile t;
+  t.lane = threadIdx.x & 63;
+  t.n = t.lane & 15;
+  t.g = t.lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wid = xcd_remap(blockIdx.x, gridDim.x) * 4 + wave;
+  t.live = wid < a.B * a.g.nstrips * a.g.nrowblk;
+  t.x0 = (wid % a.g.nstrips) * own;
+  t.y0 = ((wid / a.g.nstrips) % a.g.nrowblk) * a.g.rows;
+  const int b = wid / (a.g.nstrips * a.g.nrowblk);
+  t.y1 = min(t.y0 + a.g.rows, a.H);
+  t.ny = t.nx = 0;
+  if (t.live) extent_of(a.ext, b, a.H, a.W, t.ny, t.nx);
+  t.bytes = (uint32_t)((int64_t)a.B * a.H * a.W * kC * 2);
+  t.rowbytes = (uint32_t)a.W * kC * 2;
+  t.img = (uint32_t)b * a.H * t.rowbytes;
+  return t;
+}
+__device__ __forceinline__ const u32x4* weight_frag(const bf16* wt, const ConvTile& t, int tap, int cb) {
+  return reinterpret_cast<const u32x4*>(wt + ((tap * kC + 8 * (t.n >> 2) + 4 * cb + (t.n & 3)) * kC + 8 * t.g));
+}
+// A row's 16 B per lane to byte offset off (kOOB: dropped) of the row at so.
+// The row's offset is added to the lane's, not given in the instruction's
+// scalar offset: behind a 16-B store without one the compiler keeps the wait
+// states that the store's data registers need before they are written again.
+// With one it adds none, and where two waves share a SIMD the last lanes'
+// data was then overwritten before it was read.
+template <int ST>
+__device__ __forceinline__ void store_px(u32x4 v, rsrc_t r, uint32_t off, uint32_t so) {
+  __builtin_amdgcn_raw_buffer_store_b128(v, r, off + so, 0, ST);
+}
+// byte offset of pixel x of a row, this lane's channels; kOOB unless ok
+__device__ __forceinline__ uint32_t px_off(const ConvTile& t, int x, bool ok) {
+  return ok ? (uint32_t)(x * kC + 8 * t.g) * 2 : kOOB;
+}
+
+// One layer.  MODE 0: out = LeakyReLU(conv + bias).  MODE 1 (dgrad): out =
+// conv * (aux > 0 ? 1 : 0.01), aux = activation of the layer below (its sign
+// is the sign of its pre-activation).  Slots n hold pairs of neighbouring
+// pixels, 8 (n / 2) + 2 q + n % 2 for slot group q: an access of the wave
+// covers whole 128-B lines (interleaved by 4 n + q instead, half lines, 1500
+// x 1500 took 74 us a layer, now 60).  Tap column s of group q is then the
+// row shifted by s - 1: nine fragments a row, whose overlap is read from L1.
+template <int MODE, int ST>
+__global__ void __launch_bounds__(256, 2)
+conv3x3_kernel(const ConvArgs a) {
+  __shared__ u32x4 wl[18][64];
+  const ConvTile t = conv_tile(a, kStripPx);
+  for (int f = threadIdx.x >> 6; f < 18; f += 4) wl[f][t.lane] = *weight_frag(a.wt[0], t, f >> 1, f & 1);
+  __syncthreads();
+  if (!t.live) return;
+
+  const int xl = t.x0 + 8 * (t.n >> 1) + (t.n & 1);  // pixel of slot q: xl + 2 q
+  uint32_t ooff[4];
+  bool xin[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    ooff[q] = px_off(t, xl + 2 * q, xl + 2 * q < a.W);
+    xin[q] = xl + 2 * q < t.nx;
+  }
+  const rsrc_t rout = make_rsrc(a.out, t.bytes);
+  const int yv = t.x0 < t.nx ? min(t.y1, t.ny) : t.y0;  // rows y0 .. yv - 1 are computed
+  for (int y = max(yv, t.y0); y < t.y1; ++y) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      store_px<kStoreCached>(u32x4{0, 0, 0, 0}, rout, ooff[q], t.img + y * t.rowbytes);
+  }
+  if (yv <= t.y0) return;
+
+  float bias_r[8];
+  if constexpr (MODE == 0) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) bias_r[e] = a.bias[0][8 * t.g + e];
+  }
+  // fragment f: pixels xl + f - 1, f = 0 .. 8
+  uint32_t voff[9];
+#pragma unroll
+  for (int f = 0; f < 9; ++f) voff[f] = px_off(t, xl + f - 1, (xl + f - 1 >= 0) & (xl + f - 1 < t.nx));
+  auto load_row = [&](u32x4 (&r)[9], int y) {
+    const bool ok = (y >= 0) & (y < t.ny) & (y <= yv);
+    const rsrc_t rs = make_rsrc(a.in, ok ? t.bytes : 0u);
+    const uint32_t so = ok ? t.img + (uint32_t)y * t.rowbytes : 0u;
+#pragma unroll
+    for (int f = 0; f < 9; ++f) r[f] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff[f], so, 0);
+  };
+
+  // row y from input rows y - 1 (ra), y (rb), y + 1 (rc); loads row y + 2 into ra
+  auto step = [&](int y, u32x4 (&ra)[9], const u32x4 (&rb)[9], const u32x4 (&rc)[9]) {
+    const uint32_t so = t.img + (uint32_t)y * t.rowbytes;
+    u32x4 av[4];
+    if constexpr (MODE == 1) {
+      const rsrc_t raux = make_rsrc(a.aux, t.bytes);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) av[q] = __builtin_amdgcn_raw_buffer_load_b128(raux, ooff[q], so, 0);
+    }
+    f32x4 acc[4][2];
+#pragma unroll
+    for (int tap = 0; tap < 9; ++tap) {
+      const u32x4 (&r)[9] = tap < 3 ? ra : (tap < 6 ? rb : rc);
+      const bf16x8 w0 = as_bf16x8(wl[2 * tap][t.lane]), w1 = as_bf16x8(wl[2 * tap + 1][t.lane]);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const bf16x8 v = as_bf16x8(r[2 * q + tap % 3]);
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        acc[q][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0, v, tap == 0 ? zero : acc[q][0], 0, 0, 0);
+        acc[q][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1, v, tap == 0 ? zero : acc[q][1], 0, 0, 0);
+      }
+      if (tap == 2) {
+        load_row(ra, y + 2);
+        asm volatile("" ::: "memory");  // keeps the loads here: they would sink into the next step
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      bf16x8 h;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float v = acc[q][e >> 2][e & 3];
+        if constexpr (MODE == 0) {
+          v += bias_r[e];
+          v = fmaxf(v, 0.01f * v);
+        } else {
+          const uint32_t w = av[q][e >> 1];
+          v *= __uint_as_float((e & 1) ? (w & 0xFFFF0000u) : (w << 16)) > 0.f ? 1.f : 0.01f;
+        }
+        h[e] = f2bf(v);
+      }
+      u32x4 o = __builtin_bit_cast(u32x4, h);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = xin[q] ? o[i] : 0u;
+      store_px<ST>(o, rout, ooff[q], so);
+    }
+  };
+
+  u32x4 r0[9], r1[9], r2[9];
+  load_row(r0, t.y0 - 1);
+  load_row(r1, t.y0);
+  load_row(r2, t.y0 + 1);
+  for (int y = t.y0;; y += 3) {
+    step(y, r0, r1, r2);
+    if (y + 1 >= yv) break;
+    step(y + 1, r1, r2, r0);
+    if (y + 2 >= yv) break;
+    step(y + 2, r2, r0, r1);
+    if (y + 3 >= yv) break;
+  }
+}
+
+// lane n of each 16 receives lane n - 1's (lane n + 1's) value; 0 at the end
+__device__ __forceinline__ u32x4 px_left(u32x4 v) {
+  u32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = __builtin_amdgcn_update_dpp(0, (int)v[i], 0x111, 0xF, 0xF, true);
+  return r;
+}
+__device__ __forceinline__ u32x4 px_right(u32x4 v) {
+  u32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = __builtin_amdgcn_update_dpp(0, (int)v[i], 0x101, 0xF, 0xF, true);
+  return r;
+}
+
+// Two forward layers: the first one's rows stay in registers, three at a time
+// like the input's, and its outputs are the second layer's operand as they
+// are.  Slot n of group q is pixel 4 n + q: tap columns are other groups'
+// fragments, and the neighbours of a row's ends come from the next lane (DPP).
+// The second layer is complete on 62 of the 64 columns, and a wave computes
+// two more rows of the first layer than it owns.  Outside the extent the
+// first layer is zero, the second one's padding.
+template <int ST>
+__global__ void __launch_bounds__(256, 1)
+conv3x3_pair_kernel(const ConvArgs a) {
+  __shared__ u32x4 wl[2][18][64];
+  __shared__ __attribute__((aligned(16))) float bl[2][kC];
+  const ConvTile t = conv_tile(a, kPairPx);
+#pragma unroll
+  for (int l = 0; l < 2; ++l) {
+    for (int f = threadIdx.x >> 6; f < 18; f += 4) wl[l][f][t.lane] = *weight_frag(a.wt[l], t, f >> 1, f & 1);
+    if (threadIdx.x < kC) bl[l][threadIdx.x] = a.bias[l][threadIdx.x];
+  }
+  __syncthreads();
+  if (!t.live) return;
+  const int xl = t.x0 - 1 + 4 * t.n;  // pixel of slot q: xl + q
+  uint32_t ooff[4];
+  bool xin[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int p = 4 * t.n + q;
+    ooff[q] = px_off(t, xl + q, (p >= 1) & (p <= kPairPx) & (xl + q < a.W));
+    xin[q] = (xl + q >= 0) & (xl + q < t.nx);
+  }
+  const rsrc_t rout = make_rsrc(a.out, t.bytes);
+  const int yv = t.x0 < t.nx ? min(t.y1, t.ny) : t.y0;  // rows y0 .. yv - 1 are computed
+  for (int y = max(yv, t.y0); y < t.y1; ++y) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      store_px<kStoreCached>(u32x4{0, 0, 0, 0}, rout, ooff[q], t.img + y * t.rowbytes);
+  }
+  if (yv <= t.y0) return;
+
+  uint32_t voff[6];  // fragment f: pixels xl + f - 1
+#pragma unroll
+  for (int f = 0; f < 6; ++f) voff[f] = px_off(t, xl + f - 1, (xl + f - 1 >= 0) & (xl + f - 1 < t.nx));
+  auto load_row = [&](u32x4 (&r)[6], int y) {
+    const bool ok = (y >= 0) & (y < t.ny) & (y <= yv + 1);
+    const rsrc_t rs = make_rsrc(a.in, ok ? t.bytes : 0u);
+    const uint32_t so = ok ? t.img + (uint32_t)y * t.rowbytes : 0u;
+#pragma unroll
+    for (int f = 0; f < 6; ++f) r[f] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff[f], so, 0);
+  };
+  u32x4 r[3][6];  // input rows
+  u32x4 m[3][6];  // the first layer's rows
+#pragma unroll
+  for (int i = 0; i < 3; ++i) load_row(r[i], t.y0 - 2 + i);
+
+  // row y of layer l from its input rows; `between` runs after row ra's last use
+  auto layer = [&](int l, int y, const u32x4 (&ra)[6], const u32x4 (&rb)[6], const u32x4 (&rc)[6],
+                   u32x4 (&o)[4], auto&& between) {
+    f32x4 acc[4][2];
+#pragma unroll
+    for (int tap = 0; tap < 9; ++tap) {
+      const u32x4 (&rr)[6] = tap < 3 ? ra : (tap < 6 ? rb : rc);
+      const bf16x8 w0 = as_bf16x8(wl[l][2 * tap][t.lane]), w1 = as_bf16x8(wl[l][2 * tap + 1][t.lane]);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const bf16x8 v = as_bf16x8(rr[q + tap % 3]);
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        acc[q][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0, v, tap == 0 ? zero : acc[q][0], 0, 0, 0);
+        acc[q][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1, v, tap == 0 ? zero : acc[q][1], 0, 0, 0);
+      }
+      if (tap == 2) between();
+    }
+    const bool rv = (y >= 0) & (y < t.ny);
+    const f32x4 b01[2] = {*reinterpret_cast<const f32x4*>(&bl[l][8 * t.g]),
+                          *reinterpret_cast<const f32x4*>(&bl[l][8 * t.g + 4])};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      bf16x8 h;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float v = acc[q][e >> 2][e & 3] + b01[e >> 2][e & 3];
+        v = fmaxf(v, 0.01f * v);
+        h[e] = f2bf(v);
+      }
+      o[q] = __builtin_bit_cast(u32x4, h);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[q][i] = (xin[q] & rv) ? o[q][i] : 0u;
+    }
+  };
+  // row c of the first layer, from r[I], r[I + 1], r[I + 2], into m[I]
+  auto first = [&](int I, int c) {
+    u32x4 o[4];
+    layer(0, c, r[I], r[(I + 1) % 3], r[(I + 2) % 3], o, [&] { load_row(r[I], c + 2); });
+#pragma unroll
+    for (int q = 0; q < 4; ++q) m[I][q + 1] = o[q];
+    m[I][0] = px_left(o[3]);
+    m[I][5] = px_right(o[0]);
+  };
+  // row y of the output: the first layer's row y + 1, then the second layer
+  auto step = [&](int I, int y) {
+    first(I, y + 1);
+    u32x4 o[4];
+    layer(1, y, m[(I + 1) % 3], m[(I + 2) % 3], m[I], o, [] {});
+#pragma unroll
+    for (int q = 0; q < 4; ++q) store_px<ST>(o[q], rout, ooff[q], t.img + (uint32_t)y * t.rowbytes);
+  };
+  first(0, t.y0 - 1);
+  first(1, t.y0);
+  // whole groups of three rows as one block of instructions (the scheduler
+  // overlaps a layer's epilogue with the next one's products), then the rest
+  int y = t.y0;
+  for (; y + 3 <= yv; y += 3) {
+    step(2, y);
+    step(0, y + 1);
+    step(1, y + 2);
+  }
+  if (yv - y == 1) {
+    step(2, y);
+  } else if (yv - y == 2) {
+    step(2, y);
+    step(0, y + 1);
+  }
+}
+
+}  // namespace igm
+
+using namespace igm;
+
+namespace {
+ConvArgs conv_args(const void* in, const void* w, const float* bias, const void* aux, const int32_t* ext, int B,
+                   int H, int W, void* out, int own) {
+  ConvArgs a{};
+  a.in = (const bf16*)in;
+  a.wt[0] = (const bf16*)w;
+  a.bias[0] = bias;
+  a.aux = (const bf16*)aux;
+  a.out = (bf16*)out;
+  a.ext = ext;
+  a.B = B;
+  a.H = H;
+  a.W = W;
+  a.g = conv_geom(B, H, W, own, ext != nullptr);
+  return a;
+}
+int64_t act_bytes(int B, int H, int W) { return (int64_t)B * H * W * kC * 2; }
+// How a layer's output of so many bytes is stored.  The caches write it back
+// at the kernel's end otherwise: written through, 500 x 500 takes 8.6 us
+// instead of 10.5 and 1000 x 1000 (64 MB) 22.7 instead of 24.0.  Buffers that
+// do not stay in the 256 MB last-level cache together gain nothing from it:
+// 1500 x 1500 (144 MB, forward) took 59 to 61 us either way, and the data
+// gradient, which also reads the activation, 75.7 us with non-temporal
+// stores, 88 without (8 x 512 x 512, 134 MB: 63.9 and 71.9).  The forward
+// pass of such a batch keeps them cached (41 us, 50 non-temporal).
+inline int store_mode(int64_t bytes, bool dgrad) {
+  if (bytes <= (80 << 20)) return kStoreThrough;
+  return dgrad && bytes >= (120 << 20) ? kStoreStream : kStoreCached;
+}
+}  // namespace
+
+extern "C" {
+
+int igm_conv3x3_fwd_bf16(const void* in, const void* wpacked, const float* bias,
+                         const int32_t* extents, int32_t B, int32_t H, int32_t W, void* out,
+                         void* stream) {
+  IGM_CHECK_ARG(in && wpacked && bias && out, "null pointer");
+  IGM_CHECK_ARG(in != out, "in and out must differ");
+  IGM_CHECK_ARG(B >= 1 && H >= 1 && W >= 1 && B <= 65535, "bad sizes");
+  IGM_CHECK_ARG(act_bytes(B, H, W) < (int64_t)kOOB, "activations above 2 GiB (32-bit buffer offsets)");
+  const ConvArgs a = conv_args(in, wpacked, bias, nullptr, extents, B, H, W, out, kStripPx);
+  const dim3 grid(a.g.blocks), block(256);
+  hipStream_t st = (hipStream_t)stream;
+  switch (store_mode(act_bytes(B, H, W), false)) {
+    case kStoreThrough: hipLaunchKernelGGL((conv3x3_kernel<0, kStoreThrough>), grid, block, 0, st, a); break;
+    default: hipLaunchKernelGGL((conv3x3_kernel<0, kStoreCached>), grid, block, 0, st, a); break;
+  }
+  IGM_CHECK_LAUNCH();
+  return 0;
+}
+
+int igm_conv3x3_pair_fwd_bf16(const void* in, const void* w1, const float* b1, const void* w2,
+                              const float* b2, const int32_t* extents, int32_t B, int32_t H,
+                              int32_t W, void* out, void* stream) {
+  IGM_CHECK_ARG(in && w1 && b1 && w2 && b2 && out, "null pointer");
+  IGM_CHECK_ARG(in != out, "in and out must differ");
+  IGM_CHECK_ARG(B >= 1 && H >= 1 && W >= 1 && B <= 65535, "bad sizes");
+  IGM_CHECK_ARG(act_bytes(B, H, W) < (int64_t)kOOB, "activations above 2 GiB (32-bit buffer offsets)");
+  ConvArgs a = conv_args(in, w1, b1, nullptr, extents, B, H, W, out, kPairPx);
+  a.wt[1] = (const bf16*)w2;
+  a.bias[1] = b2;
+  const dim3 grid(a.g.blocks), block(256);
+  hipStream_t st = (hipStream_t)stream;
+  switch (store_mode(act_bytes(B, H, W), false)) {
+    case kStoreThrough: hipLaunchKernelGGL((conv3x3_pair_kernel<kStoreThrough>), grid, block, 0, st, a); break;
+    default: hipLaunchKernelGGL((conv3x3_pair_kernel<kStoreCached>), grid, block, 0, st, a); break;
+  }
+  IGM_CHECK_LAUNCH();
+  return 0;
+}
+
+int igm_conv3x3_dgrad_bf16(const void* dz, const void* wpacked_dgrad, const void* act_below,
+                           const int32_t* extents, int32_t B, int32_t H, int32_t W, void* dz_below,
+                           void* stream) {
+  IGM_CHECK_ARG(dz && wpacked_dgrad && act_below && dz_below, "null pointer");
+  IGM_CHECK_ARG(dz != dz_below, "in and out must differ");
+  IGM_CHECK_ARG(B >= 1 && H >= 1 && W >= 1 && B <= 65535, "bad sizes");
+  IGM_CHECK_ARG(act_bytes(B, H, W) < (int64_t)kOOB, "activations above 2 GiB (32-bit buffer offsets)");
+  const ConvArgs a = conv_args(dz, wpacked_dgrad, nullptr, act_below, extents, B, H, W, dz_below, kStripPx);
+  const dim3 grid(a.g.blocks), block(256);
+  hipStream_t st = (hipStream_t)stream;
+  switch (store_mode(act_bytes(B, H, W), true)) {
+    case kStoreThrough: hipLaunchKernelGGL((conv3x3_kernel<1, kStoreThrough>), grid, block, 0, st, a); break;
+    case kStoreStream: hipLaunchKernelGGL((conv3x3_kernel<1, kStoreStream>), grid, block, 0, st, a); break;
+    default: hipLaunchKernelGGL((conv3x3_kernel<1, kStoreCached>), grid, block, 0, st, a); break;
+  }
+  IGM_CHECK_LAUNCH();
+  return 0;
+}
+
+}  // extern "C"

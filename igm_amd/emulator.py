@@ -115,19 +115,21 @@ class CNN:
         L.call("igm_conv_in_fwd", *fptrs, fb, fr, fc, ext, B, H, W, L.ptr(self.kernel(0)),
                L.ptr(self.bias(0)), L.ptr(act), st)
         acts = [act]
-        spare = None
-        for li in range(1, self.nl):
-            if keep or spare is None:
-                out = torch.empty_like(act)
-            else:
-                out = spare
-            L.call("igm_conv3x3_fwd_bf16", L.ptr(act), L.ptr(self.fwd[li - 1]), L.ptr(self.bias(li)),
-                   ext, B, H, W, L.ptr(out), st)
+        other = None
+        li = 1
+        while li < self.nl:
+            out = torch.empty_like(act) if keep or other is None else other
+            if keep or li + 1 == self.nl:
+                L.call("igm_conv3x3_fwd_bf16", L.ptr(act), L.ptr(self.fwd[li - 1]), L.ptr(self.bias(li)),
+                       ext, B, H, W, L.ptr(out), st)
+                li += 1
+            else:  # two layers in one launch: the one between them is not stored
+                L.call("igm_conv3x3_pair_fwd_bf16", L.ptr(act), L.ptr(self.fwd[li - 1]), L.ptr(self.bias(li)),
+                       L.ptr(self.fwd[li]), L.ptr(self.bias(li + 1)), ext, B, H, W, L.ptr(out), st)
+                li += 2
             if keep:
                 acts.append(out)
-            else:
-                spare = act
-            act = out
+            act, other = out, act
         Y = torch.empty((B, H, W, self.cout), dtype=torch.float32, device=dev)
         L.call("igm_conv1x1_head_fwd", L.ptr(act), L.ptr(self.head), L.ptr(self.bias(self.nl)), ext,
                B, H, W, self.cout, L.ptr(Y), st)

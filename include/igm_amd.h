@@ -263,6 +263,13 @@ int igm_conv3x3_fwd_bf16(const void* in, const void* wpacked, const float* bias,
                          const int32_t* extents, int32_t B, int32_t H, int32_t W, void* out,
                          void* stream);
 
+/* Two such layers in one launch: layer (w1, b1), then layer (w2, b2), bit for
+ * bit what two igm_conv3x3_fwd_bf16 calls give.  The first layer's output is
+ * not stored. */
+int igm_conv3x3_pair_fwd_bf16(const void* in, const void* w1, const float* b1, const void* w2,
+                              const float* b2, const int32_t* extents, int32_t B, int32_t H,
+                              int32_t W, void* out, void* stream);
+
 /* Input gradient of a 3x3 layer (the tape through Conv2D, emulate.py:252):
  * dz_below = conv(dz, flipped W) * LeakyReLU'(act_below).
  * wpacked_dgrad: [9][32 in][32 out] bf16 with the taps reversed. */

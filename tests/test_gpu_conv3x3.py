@@ -1,0 +1,91 @@
+"""The 3x3 layer kernels (igm_conv3x3_fwd_bf16, igm_conv3x3_dgrad_bf16,
+igm_conv3x3_pair_fwd_bf16) element by element against float64 sums of the
+same bf16 operands, at the edges of their 62- and 64-column strips and row
+blocks, on padded batches, and where two blocks share a compute unit.
+
+Tolerance of an element: half a bf16 step of the result, 2^-9 |ref| (2^-8 is
+asked), and the float32 accumulation of 288 products, at most 288 * 2^-24 *
+sum |w x| ~ 288 * 6e-8 * 14 = 2.4e-4 (3e-4).  Two layers in one launch run
+the same instructions as two launches: equal bits."""
+import pytest
+import torch
+
+from igm_amd import _lib as L
+
+pytestmark = pytest.mark.gpu
+
+# (B, H, W, extents): one pixel, strips of 62 and 64 columns and one more,
+# 1 to 8 rows, batches with uneven and empty entries, and grids of more than
+# 1024 waves (blocks of at most 32 rows: 8 x 600 x 700) and of long waves
+CASES = [(1, 1, 1, None), (1, 2, 62, None), (1, 3, 63, None), (1, 4, 64, None), (1, 5, 65, None), (1, 7, 125, None),
+         (1, 8, 129, None), (1, 131, 124, None), (3, 37, 131, [(37, 131), (20, 64), (1, 1)]),
+         (2, 65, 70, [(65, 5), (33, 70)]), (8, 600, 700, [(600 - 61 * i, 700 - 83 * i) for i in range(8)]),
+         (1, 1100, 1300, None)]
+
+
+def case(B, H, W, dev):
+    g = torch.Generator().manual_seed(B + 7 * H + W)
+    x = torch.randn((B, H, W, 32), generator=g).to(torch.bfloat16).to(dev)
+    ws = [(torch.randn((9, 32, 32), generator=g) * 0.06).to(torch.bfloat16).to(dev) for _ in range(2)]
+    bs = [(torch.randn(32, generator=g) * 0.1).to(dev) for _ in range(2)]
+    return x, ws, bs
+
+
+def conv64(x, w):
+    """"Same" correlation, float64: w [tap][out][in]."""
+    B, H, W, C = x.shape
+    xp = torch.nn.functional.pad(x.double(), (0, 0, 1, 1, 1, 1))
+    out = torch.zeros((B, H, W, C), dtype=torch.float64, device=x.device)
+    for t in range(9):
+        r, s = t // 3, t % 3
+        out += (xp[:, r:r + H, s:s + W].reshape(-1, C) @ w[t].double().t().contiguous()).view(B, H, W, C)
+    return out
+
+
+def masked(x, ext):
+    """x with zeros outside each entry's extent."""
+    if ext is None:
+        return x
+    y = torch.zeros_like(x)
+    for b, (ny, nx) in enumerate(ext):
+        y[b, :ny, :nx] = x[b, :ny, :nx]
+    return y
+
+
+def check(out, ref):
+    d = (out.double() - ref).abs() - (2.0 ** -8 * ref.abs() + 3e-4)
+    assert bool(torch.isfinite(out.float()).all())
+    assert float(d.max()) <= 0, (float(d.max()), int((d > 0).sum()))
+
+
+@pytest.mark.parametrize("B,H,W,ext", CASES)
+def test_layers_against_float64(dev, B, H, W, ext):
+    print(f"case conv3x3 {B} x {H} x {W}", flush=True)
+    x, (w1, w2), (b1, b2) = case(B, H, W, dev)
+    e = None if ext is None else torch.tensor(ext, dtype=torch.int32, device=dev)
+    st = L.stream_ptr()
+    one, two, both, dg = (torch.full_like(x, float("nan")) for _ in range(4))
+    L.call("igm_conv3x3_fwd_bf16", L.ptr(x), L.ptr(w1), L.ptr(b1), L.ptr(e), B, H, W, L.ptr(one), st)
+    L.call("igm_conv3x3_fwd_bf16", L.ptr(one), L.ptr(w2), L.ptr(b2), L.ptr(e), B, H, W, L.ptr(two), st)
+    L.call("igm_conv3x3_pair_fwd_bf16", L.ptr(x), L.ptr(w1), L.ptr(b1), L.ptr(w2), L.ptr(b2), L.ptr(e), B, H, W,
+           L.ptr(both), st)
+    L.call("igm_conv3x3_dgrad_bf16", L.ptr(x), L.ptr(w1), L.ptr(two), L.ptr(e), B, H, W, L.ptr(dg), st)
+    torch.cuda.synchronize()
+    xm = masked(x, ext)
+    z = conv64(xm, w1)
+    check(one, masked(torch.nn.functional.leaky_relu(z + b1.double(), 0.01), ext))
+    check(dg, masked(z * torch.where(two.float() > 0, 1.0, 0.01), ext))
+    assert torch.equal(both.view(torch.int16), two.view(torch.int16))
+
+
+def test_network_forward_equals_layer_by_layer(dev):
+    """CNN.forward in launches of two layers gives the bits of the pass that
+    keeps every activation, for even and odd counts of 3x3 layers."""
+    from igm_amd import emulator as EM
+    for nl in (1, 2, 3, 4, 5):
+        cnn = EM.CNN(nz=5, nb_layers=nl, device=dev, seed=nl)
+        X = torch.randn((2, 33, 71, 5), generator=torch.Generator().manual_seed(nl)).to(dev)
+        fields = EM.nhwc_fields(X)
+        Y, acts = cnn.forward(fields, keep=True)
+        assert len(acts) == nl
+        assert torch.equal(cnn.forward(fields), Y)
