@@ -26,4 +26,8 @@ __device__ __forceinline__ void extent_of(const int32_t* ext, int b, int H, int 
   nx = ext ? min(ext[2 * b + 1], W) : W;
 }
 
+// Per-block partial sums of a 3x3 layer's weight gradient (wgrad3x3.hip).
+int wgrad3x3_launch(const void* act, const void* dz, const int32_t* ext, int B, int H, int W, int nblocks,
+                    float* partials, int accumulate, hipStream_t st);
+
 }  // namespace igm

@@ -1,0 +1,182 @@
+// Weight gradient of the emulator's 32 -> 32 3x3 layers on gfx950:
+//   dW[tap][co][ci] = sum_p dz[p][co] * act[p + delta_tap][ci],  db[co] = sum_p dz[p][co]
+// (the tape through Conv2D, emulate/emulate.py:252).
+//
+// K is the pixels: a product takes 16 co x 16 ci over 32 pixels, so both
+// operands have to be transposed, 8 pixels of one channel per lane where NHWC
+// rows hold 8 channels of one pixel.  A wave owns a strip of 32 columns, walks
+// down its rows and keeps the whole 9 x 32 x 32 gradient in its accumulators
+// (144 registers per lane).  Each row of either operand is read from memory
+// once, written to LDS as it is and read back transposed (ds_read_b64_tr_b16):
+// the three x-shifts of the activation are three reads at other pixels, and
+// their fragments stay in registers for the three rows that use them.  The
+// wave's LDS is its own, so nothing waits for a barrier, and no VALU work is
+// left.  db is a product with ones.
+//
+// What bounds it: 1000 x 1000 takes 25.5 us, 128 MB at 5.0 TB/s, a copy's
+// rate (36 products of 16 cycles per 32 pixels are 7.5 us); 8 x 496 x 496
+// padded patches 40 us.  The earlier kernel transposed with VALU packing into
+// block-wide LDS tiles, read by all waves between barriers: 39 and 62 us.
+#include "conv_common.hpp"
+
+namespace igm {
+
+constexpr int kWgPx = 32;                 // columns of a wave's strip: the K of one product
+constexpr int kWgEntries = 9 * kC * kC + kC;  // floats of a block's partial sums
+constexpr int kRing = 4;  // rows of each operand in flight from memory
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+
+__global__ void __launch_bounds__(256, 1)
+wgrad3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const int32_t* __restrict__ ext,
+                int B, int H, int W, int nstrips, int nchunk, int rows, int accumulate,
+                float* __restrict__ partials) {
+  // rows in transposition, later the waves' sums
+  constexpr int kStage = (kWgPx + 16 + kWgPx) * kC;
+  __shared__ __attribute__((aligned(16))) union {
+    bf16 rows[4][kStage];
+    f32x4 sums[4][kWgEntries / 4];
+  } sm;
+  const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  bf16* sa = sm.rows[wave];                       // activation row: pixels x0 - 1 .. x0 + 32
+  bf16* sz = sa + (kWgPx + 16) * kC;       // dz row: pixels x0 .. x0 + 31
+  const uint32_t bytes = (uint32_t)((int64_t)B * H * W * kC * 2);
+  const uint32_t rowbytes = (uint32_t)W * kC * 2;
+
+  f32x4 acc[9][2][2], accb[2];
+#pragma unroll
+  for (int t = 0; t < 9; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[t][i >> 1][i & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  accb[0] = accb[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  bf16x8 ones;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) ones[e] = f2bf(1.f);
+
+  // transposed operand: 32 pixels (from pixel p) of channel 16 cb + n; slot
+  // 8 g + j is pixel 4 g + j (j < 4) or 16 + 4 g + j - 4
+  auto frag = [&](const bf16* s, int p, int cb) {
+    const bf16* q = s + (p + 4 * g + (n >> 2)) * kC + 16 * cb + 4 * (n & 3);
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)q);
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(q + 16 * kC));
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+
+  const int ntask = B * nstrips * nchunk;
+  for (int task = blockIdx.x * 4 + wave; task < ntask; task += gridDim.x * 4) {
+    const int x0 = (task % nstrips) * kWgPx;
+    const int y0 = ((task / nstrips) % nchunk) * rows;
+    const int b = task / (nstrips * nchunk);
+    int ny, nx;
+    extent_of(ext, b, H, W, ny, nx);
+    const int y1 = min(y0 + rows, ny);
+    if (x0 >= nx || y0 >= y1) continue;
+    const uint32_t img = (uint32_t)b * H * rowbytes;
+    // a lane's 16 B of a row: pixel lane / 4 of 16, chunk lane % 4
+    const int px = lane >> 2;
+    auto off = [&](int x, bool ok) { return (ok & (x >= 0) & (x < nx)) ? (uint32_t)(x * kC * 2 + (lane & 3) * 16) : kOOB; };
+    const uint32_t oz[2] = {off(x0 + px, true), off(x0 + 16 + px, true)};
+    const uint32_t oa[3] = {off(x0 - 1 + px, true), off(x0 + 15 + px, true), off(x0 + 31 + px, px < 2)};
+    u32x4 stz[kRing][2], sta[kRing][3];
+    // feed j: activation row y0 - 1 + j and dz row y0 - 2 + j
+    auto load = [&](int s, int j) {
+      const int ya = y0 - 1 + j, yz = y0 - 2 + j;
+      const bool oka = (ya >= 0) & (ya < ny) & (ya <= y1), okz = (yz >= y0) & (yz < y1);
+      const rsrc_t ra = make_rsrc(act, oka ? bytes : 0u), rz = make_rsrc(dz, okz ? bytes : 0u);
+      const uint32_t pa = oka ? img + (uint32_t)ya * rowbytes : 0u, pz = okz ? img + (uint32_t)yz * rowbytes : 0u;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) sta[s][i] = __builtin_amdgcn_raw_buffer_load_b128(ra, oa[i], pa, 0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) stz[s][i] = __builtin_amdgcn_raw_buffer_load_b128(rz, oz[i], pz, 0);
+    };
+    bf16x8 F[4][3][2], D[2][2];
+    auto feed = [&](int s, int f, int d, int j) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x4*>(sa + i * 16 * kC + lane * 8) = sta[s][i];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) *reinterpret_cast<u32x4*>(sz + i * 16 * kC + lane * 8) = stz[s][i];
+      load(s, j + kRing);
+#pragma unroll
+      for (int t = 0; t < 3; ++t)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) F[f][t][c] = frag(sa, t, c);
+#pragma unroll
+      for (int c = 0; c < 2; ++c) D[d][c] = frag(sz, 0, c);
+    };
+    // products of dz row y0 + j - 3, whose operands feeds j - 3 .. j - 1 read
+    auto mult = [&](int j) {
+#pragma unroll
+      for (int t = 0; t < 9; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          acc[t][i >> 1][i & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              D[(j + 1) & 1][i >> 1], F[(j + 1 + t / 3) & 3][t % 3][i & 1], acc[t][i >> 1][i & 1], 0, 0, 0);
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        accb[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(D[(j + 1) & 1][c], ones, accb[c], 0, 0, 0);
+    };
+#pragma unroll
+    for (int s = 0; s < kRing; ++s) load(s, s);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) feed(j % kRing, j & 3, j & 1, j);
+    const int end = y1 - y0 + 3;
+    // four steps at a time (the rings' period); rows past the last feed zeros
+    for (int j = 3; j < end; j += 4) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        feed((3 + k) % kRing, (3 + k) & 3, (3 + k) & 1, j + k);
+        mult(3 + k);
+      }
+    }
+  }
+
+  // the four waves' sums, in order, in the lanes' own layout: entry
+  // ((tap * 4 + block) * 64 + lane) * 4 + e, then the bias
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < 9; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sm.sums[wave][(t * 4 + i) * 64 + lane] = acc[t][i >> 1][i & 1];
+  if (n == 0) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) sm.sums[wave][9 * kC * kC / 4 + 4 * c + g] = accb[c];
+  }
+  __syncthreads();
+  f32x4* P = reinterpret_cast<f32x4*>(partials + (int64_t)blockIdx.x * kWgEntries);
+  constexpr int kPer = (kWgEntries / 4 + 255) / 256;
+  f32x4 prev[kPer];
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    const int q = threadIdx.x + 256 * k;
+    prev[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (accumulate) prev[k] = P[q < kWgEntries / 4 ? q : 0];
+  }
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    const int q = threadIdx.x + 256 * k;
+    if (q < kWgEntries / 4) {
+      const f32x4 v = ((sm.sums[0][q] + sm.sums[1][q]) + sm.sums[2][q]) + sm.sums[3][q];
+      P[q] = accumulate ? prev[k] + v : v;
+    }
+  }
+}
+
+int wgrad3x3_launch(const void* act, const void* dz, const int32_t* ext, int B, int H, int W, int nblocks,
+                    float* partials, int accumulate, hipStream_t st) {
+  const int nstrips = (W + kWgPx - 1) / kWgPx;
+  const int64_t waves = 4 * (int64_t)nblocks;
+  // Equal shares for all waves, in multiples of the four steps of the loop; at
+  // most 32 rows in a batch of uneven entries, whose padding is skipped.
+  int64_t rows = ((int64_t)B * nstrips * H + waves - 1) / waves;
+  rows = (rows + 3) / 4 * 4;
+  if (ext && rows > 32) rows = 32;
+  const int nchunk = (int)((H + rows - 1) / rows);
+  hipLaunchKernelGGL(wgrad3x3_kernel, dim3(nblocks), dim3(256), 0, st, (const bf16*)act, (const bf16*)dz, ext, B, H, W,
+                     nstrips, nchunk, (int)rows, accumulate, partials);
+  IGM_CHECK_LAUNCH();
+  return 0;
+}
+
+}  // namespace igm

@@ -333,6 +333,17 @@ int igm_conv_in_wgrad_partials(const float* f0, const float* f1, const float* f2
 int igm_conv_wgrad_reduce_f32(int32_t taps, int32_t cout, int32_t nblocks, float* partials,
                               int32_t accumulate, float* dW_hwio, float* db, void* stream);
 
+/* The reduction of every layer of a network in one launch: the partial sums
+ * of layer 1 (nblocks_in rows), of the nlayers3x3 3x3 layers (nblocks_3x3 rows
+ * each, one layer's workspace after the other) and of the output layer
+ * (nblocks_head rows, cout channels) into the flat gradient g, whose layer l
+ * has its kernel (HWIO) at g + offs[2 l] and its bias at g + offs[2 l + 1]
+ * (offs: device).  A fixed order; the partial sums are not changed. */
+int igm_wgrad_reduce_layers_f32(int32_t nlayers3x3, int32_t cout, int32_t nblocks_in,
+                                int32_t nblocks_3x3, int32_t nblocks_head, const float* part_in,
+                                const float* part_3x3, const float* part_head, int32_t accumulate,
+                                const int64_t* offs, float* g, void* stream);
+
 /* Gradient of the emulator with respect to its 5 input fields (the tape
  * gradient through the network of data_assimilation/optimize/update.py:29-73),
  * through layer 1: dX (fp32 NHWC [B][H][W][5]) from dz1, the bf16 gradient at

@@ -89,3 +89,30 @@ def test_network_forward_equals_layer_by_layer(dev):
         Y, acts = cnn.forward(fields, keep=True)
         assert len(acts) == nl
         assert torch.equal(cnn.forward(fields), Y)
+
+
+@pytest.mark.parametrize("nblocks,accumulate", [(1, 0), (3, 1), (256, 0), (512, 1)])
+@pytest.mark.parametrize("B,H,W,ext", [(1, 1, 1, None), (1, 5, 33, None), (2, 13, 64, [(13, 31), (7, 64)]),
+                                       (3, 66, 70, [(65, 70), (66, 5), (1, 1)]), (1, 300, 257, None)])
+def test_weight_gradient_against_float64(dev, B, H, W, ext, nblocks, accumulate):
+    """igm_conv_wgrad_bf16 for any number of partial-sum rows, fewer and more
+    than there is work for.  Tolerance: products of 32 pixels are added in
+    float32 chains of at most 77,100 / 32 / 4 = 600 links (one block of four
+    waves); if every rounding went the same way, 600 * 2^-24 = 3.6e-5 of the
+    terms' size, as a random walk 1.5e-6: 1e-5 of the result's norm."""
+    x, (w, z2), (b, _) = case(B, H, W, dev)
+    dz = torch.randn((B, H, W, 32), generator=torch.Generator().manual_seed(H)).to(torch.bfloat16).to(dev)
+    e = None if ext is None else torch.tensor(ext, dtype=torch.int32, device=dev)
+    ws = torch.full((L.load().igm_wgrad_workspace_floats(9, nblocks),), float("nan"), device=dev)
+    dW, db = torch.ones((3, 3, 32, 32), device=dev), torch.ones(32, device=dev)
+    L.call("igm_conv_wgrad_bf16", 9, L.ptr(x), L.ptr(dz), L.ptr(e), B, H, W, 32, nblocks, L.ptr(ws), accumulate,
+           L.ptr(dW), L.ptr(db), L.stream_ptr())
+    torch.cuda.synchronize()
+    xp = torch.nn.functional.pad(masked(x, ext).double(), (0, 0, 1, 1, 1, 1))
+    zm = masked(dz, ext).double().reshape(-1, 32)
+    for t in range(9):
+        ref = xp[:, t // 3:t // 3 + H, t % 3:t % 3 + W].reshape(-1, 32).t().contiguous() @ zm + accumulate
+        d = torch.linalg.vector_norm(dW[t // 3, t % 3].double() - ref)
+        assert float(d) <= 1e-5 * max(float(torch.linalg.vector_norm(ref)), 1.0), (t, float(d))
+    ref = zm.sum(0) + accumulate
+    assert float(torch.linalg.vector_norm(db.double() - ref)) <= 1e-5 * max(float(torch.linalg.vector_norm(ref)), 1.0)
