@@ -15,12 +15,11 @@
 //  head_mfma_kernel     1x1 32 -> 2Nz (<= 32) output layer, fp32 out.
 //  wgrad1x1_kernel      weight gradient of the head: K = pixels; tiles are
 //                       transposed into LDS as [channel][pixel]; per-block
-//                       partial sums.  (3x3 layers: wgrad3x3.hip)
+//                       partial sums.  (3x3 layers and layer 1: wgrad3x3.hip)
 //  wgrad_reduce_*       deterministic sums of the partials: every layer of a
 //                       network in one launch, or one layer in two stages.
 //  head_bwd_kernel      dY -> dA16 * LeakyReLU'(A16) (fp32 VALU) and a padded
 //                       bf16 copy of dY for the head's wgrad.
-//  conv_in_wgrad_kernel layer-1 weight gradient, fp32 VALU.
 //  Adam: per-tensor clip_by_norm + legacy Adam on the fp32 master weights,
 //  then bf16 packing of the MFMA operands.
 #include "conv_common.hpp"
@@ -561,120 +560,7 @@ inline void group_rows(int nblk, int* R, int* G) {
   *G = (nblk + *R - 1) / *R;
 }
 
-// ------------------------------------------------------ layer-1 wgrad --
-// dW1[r][s][ci][co] (HWIO, fp32) = sum_p X[p + delta][ci] * dZ1[p][co]; db1.
-// Persistent blocks over tiles of 4 rows x 64 pixels; wave w takes row w of
-// a tile.  Lane l accumulates a 6 x 4 register tile of the output: the
-// (tap, ci) pairs m = 6 (l / 8) .. +5 (m = tap * 5 + ci; 48 slots, the last
-// three empty) by the output channels co = 4 (l % 8) .. +3.  Per pixel, six
-// LDS reads of X and one 16-B read of dZ feed 24 FMAs.  At the end the four
-// waves' tiles are summed in wave order into partials[blk][1440 + 32]
-// (P[m * 32 + co], then the 32 bias sums).
-constexpr int kWgTileW = 64, kWgTileH = 4;
-constexpr int kWgOut = 9 * kCin * kC + kC;  // 1472 partial entries per block
-__global__ void __launch_bounds__(256)
-conv_in_wgrad_kernel(const float* __restrict__ f0, const float* __restrict__ f1,
-                     const float* __restrict__ f2, const float* __restrict__ f3,
-                     const float* __restrict__ f4, int64_t fb, int64_t fr, int64_t fc,
-                     const int32_t* __restrict__ ext, int B, int H, int W,
-                     const bf16* __restrict__ dz, int accumulate, float* __restrict__ partials) {
-  __shared__ float xs[kWgTileH + 2][kWgTileW + 2][kCin];
-  __shared__ float4 dzs[kWgTileH][kWgTileW][kC / 4];
-  __shared__ float red[4][kWgOut];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int mb = lane >> 3, nb = lane & 7;
-  const float* fs[kCin] = {f0, f1, f2, f3, f4};
-  float acc[6][4], dbacc[4] = {0.f, 0.f, 0.f, 0.f};
-  int xoff[6];  // LDS offset of the lane's (tap, ci) pairs from xs[w][px][0]
-#pragma unroll
-  for (int j = 0; j < 6; ++j) {
-    const int m = min(6 * mb + j, 9 * kCin - 1), tap = m / kCin, ci = m % kCin;
-    xoff[j] = ((tap / 3) * (kWgTileW + 2) + tap % 3) * kCin + ci;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) acc[j][q] = 0.f;
-  }
-  const int ntx = (W + kWgTileW - 1) / kWgTileW, nty = (H + kWgTileH - 1) / kWgTileH;
-  const int ntiles = B * nty * ntx;  // < 2^25: layer-1 gradient below 2 GiB
-  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int b = tile / (nty * ntx);
-    const int y0 = ((tile / ntx) % nty) * kWgTileH;
-    const int x0 = (tile % ntx) * kWgTileW;
-    int ny, nx;
-    extent_of(ext, b, H, W, ny, nx);
-    if (y0 >= ny || x0 >= nx) continue;
-    __syncthreads();
-    // X with a one-pixel halo, zero outside the entry's extent
-    for (int c = tid; c < (kWgTileH + 2) * (kWgTileW + 2) * kCin; c += 256) {
-      const int ci = c % kCin, t = (c / kCin) % (kWgTileW + 2), row = c / (kCin * (kWgTileW + 2));
-      const int yy = y0 - 1 + row, xx = x0 - 1 + t;
-      float v = 0.f;
-      if (yy >= 0 && yy < ny && xx >= 0 && xx < nx)
-        v = fs[ci][(int64_t)b * fb + (int64_t)yy * fr + (int64_t)xx * fc];
-      xs[row][t][ci] = v;
-    }
-    // dZ1 (bf16, 32 channels), zero outside the extent
-    for (int c = tid; c < kWgTileH * kWgTileW * 4; c += 256) {
-      const int chunk = c & 3, px = (c >> 2) % kWgTileW, row = (c >> 2) / kWgTileW;
-      const int y = y0 + row, x = x0 + px;
-      bf16x8 v;
-      if (y < ny && x < nx) {
-        v = *reinterpret_cast<const bf16x8*>(dz + (((int64_t)b * H + y) * W + x) * kC + chunk * 8);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = f2bf(0.f);
-      }
-      dzs[row][px][2 * chunk] = make_float4(bf2f(v[0]), bf2f(v[1]), bf2f(v[2]), bf2f(v[3]));
-      dzs[row][px][2 * chunk + 1] = make_float4(bf2f(v[4]), bf2f(v[5]), bf2f(v[6]), bf2f(v[7]));
-    }
-    __syncthreads();
-    const float* xw = &xs[w][0][0];
-    for (int px = 0; px < kWgTileW; ++px) {
-      const float4 d = dzs[w][px][nb];
-      dbacc[0] += d.x;
-      dbacc[1] += d.y;
-      dbacc[2] += d.z;
-      dbacc[3] += d.w;
-#pragma unroll
-      for (int j = 0; j < 6; ++j) {
-        const float xv = xw[px * kCin + xoff[j]];
-        acc[j][0] += xv * d.x;
-        acc[j][1] += xv * d.y;
-        acc[j][2] += xv * d.z;
-        acc[j][3] += xv * d.w;
-      }
-    }
-  }
-  // the four waves' tiles, summed in wave order
-#pragma unroll
-  for (int j = 0; j < 6; ++j) {
-    const int m = 6 * mb + j;
-    if (m < 9 * kCin) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) red[w][m * kC + 4 * nb + q] = acc[j][q];
-    }
-  }
-  if (mb == 0) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) red[w][9 * kCin * kC + 4 * nb + q] = dbacc[q];
-  }
-  __syncthreads();
-  float* P = partials + (int64_t)blockIdx.x * kWgOut;
-  constexpr int kPer = (kWgOut + 255) / 256;
-  float prev[kPer];  // (all loads before the first store)
-#pragma unroll
-  for (int k = 0; k < kPer; ++k) {
-    const int i = tid + 256 * k;
-    prev[k] = (accumulate && i < kWgOut) ? P[i] : 0.f;
-  }
-#pragma unroll
-  for (int k = 0; k < kPer; ++k) {
-    const int i = tid + 256 * k;
-    if (i < kWgOut) {
-      const float v = ((red[0][i] + red[1][i]) + red[2][i]) + red[3][i];
-      P[i] = accumulate ? prev[k] + v : v;
-    }
-  }
-}
+constexpr int kWgOut = 9 * kCin * kC + kC;  // floats of a block's partial sums of layer 1 (wgrad3x3.hip)
 
 // Stage 2 as a plain column sum: out[i] = sum over the group rows of P[.][i],
 // i < count
@@ -828,21 +714,6 @@ int igm_conv_wgrad_partials_bf16(int32_t taps, const void* act, const void* dz,
   if (taps == 9) return wgrad3x3_launch(act, dz, extents, B, H, W, nblocks, partials, acc, st);
   hipLaunchKernelGGL(wgrad1x1_kernel, dim3(nblocks), dim3(256), 0, st, (const bf16*)act, (const bf16*)dz,
                      extents, B, H, W, acc, partials);
-  IGM_CHECK_LAUNCH();
-  return 0;
-}
-
-int igm_conv_in_wgrad_partials(const float* f0, const float* f1, const float* f2, const float* f3,
-                               const float* f4, int64_t fb, int64_t fr, int64_t fc,
-                               const int32_t* extents, int32_t B, int32_t H, int32_t W,
-                               const void* dz1, int32_t nblocks, float* partials,
-                               int32_t accumulate, void* stream) {
-  IGM_CHECK_ARG(f0 && f1 && f2 && f3 && f4 && dz1 && partials, "null pointer");
-  IGM_CHECK_ARG(nblocks >= 1 && B >= 1 && H >= 1 && W >= 1, "bad sizes");
-  IGM_CHECK_ARG((int64_t)B * H * W * kC * 2 < (int64_t)kOOB, "activations above 2 GiB (32-bit buffer offsets)");
-  hipLaunchKernelGGL(conv_in_wgrad_kernel, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, f0,
-                     f1, f2, f3, f4, fb, fr, fc, extents, B, H, W, (const bf16*)dz1,
-                     accumulate ? 1 : 0, partials);
   IGM_CHECK_LAUNCH();
   return 0;
 }

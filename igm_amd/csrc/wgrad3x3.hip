@@ -1,4 +1,5 @@
-// Weight gradient of the emulator's 32 -> 32 3x3 layers on gfx950:
+// Weight gradients of the emulator's 3x3 layers on gfx950 (layer 1, which reads
+// float32 fields: below).  32 -> 32 layers:
 //   dW[tap][co][ci] = sum_p dz[p][co] * act[p + delta_tap][ci],  db[co] = sum_p dz[p][co]
 // (the tape through Conv2D, emulate/emulate.py:252).
 //
@@ -28,6 +29,18 @@ constexpr int kRing = 4;  // rows of each operand in flight from memory
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
+// Transposed operand from LDS rows of kCh channels per pixel: 32 pixels, from
+// pixel p on, of channel 16 cb + lane % 16; with g = lane / 16, slot 8 g + j
+// is pixel 4 g + j (j < 4) or 16 + 4 g + j - 4.
+template <int kCh>
+__device__ __forceinline__ bf16x8 transposed(const bf16* s, int p, int cb) {
+  const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+  const bf16* q = s + (p + 4 * g + (n >> 2)) * kCh + 16 * cb + 4 * (n & 3);
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)q);
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(q + 16 * kCh));
+  return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
 __global__ void __launch_bounds__(256, 1)
 wgrad3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const int32_t* __restrict__ ext,
                 int B, int H, int W, int nstrips, int nchunk, int rows, int accumulate,
@@ -54,15 +67,6 @@ wgrad3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const
   bf16x8 ones;
 #pragma unroll
   for (int e = 0; e < 8; ++e) ones[e] = f2bf(1.f);
-
-  // transposed operand: 32 pixels (from pixel p) of channel 16 cb + n; slot
-  // 8 g + j is pixel 4 g + j (j < 4) or 16 + 4 g + j - 4
-  auto frag = [&](const bf16* s, int p, int cb) {
-    const bf16* q = s + (p + 4 * g + (n >> 2)) * kC + 16 * cb + 4 * (n & 3);
-    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)q);
-    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(q + 16 * kC));
-    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-  };
 
   const int ntask = B * nstrips * nchunk;
   for (int task = blockIdx.x * 4 + wave; task < ntask; task += gridDim.x * 4) {
@@ -101,9 +105,9 @@ wgrad3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const
 #pragma unroll
       for (int t = 0; t < 3; ++t)
 #pragma unroll
-        for (int c = 0; c < 2; ++c) F[f][t][c] = frag(sa, t, c);
+        for (int c = 0; c < 2; ++c) F[f][t][c] = transposed<kC>(sa, t, c);
 #pragma unroll
-      for (int c = 0; c < 2; ++c) D[d][c] = frag(sz, 0, c);
+      for (int c = 0; c < 2; ++c) D[d][c] = transposed<kC>(sz, 0, c);
     };
     // products of dz row y0 + j - 3, whose operands feeds j - 3 .. j - 1 read
     auto mult = [&](int j) {
@@ -163,20 +167,197 @@ wgrad3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const
   }
 }
 
-int wgrad3x3_launch(const void* act, const void* dz, const int32_t* ext, int B, int H, int W, int nblocks,
-                    float* partials, int accumulate, hipStream_t st) {
-  const int nstrips = (W + kWgPx - 1) / kWgPx;
+// Layer 1 (5 float32 fields -> 32): dW1[tap][ci][co] = sum_p X[p + delta_tap][ci] * dz1[p][co].
+//
+// The same march on the matrix units, with every float32 input split into
+// three bf16 parts, x = h + m + l: 8 + 8 + 8 significant bits are all 24 of
+// them, so the parts' products with the bf16 dz1 are exact and the sums stay
+// float32, one per part.  The 5 fields' parts and a one are the 16 rows of a
+// product: two products per tap and 32 pixels, the bias with them.  Channel
+// 4 i + e of a pixel: part e (h, m, l) of field i for e < 3; e = 3: field 4's
+// h, m, l, then the one.
+//
+// What bounds it: 1000 x 1000 takes 21 us (512 blocks, 23 with 256), 84 MB at
+// 4.0 TB/s; 8 x 496 x 496 padded patches 30 us.  Float32 FMAs from LDS tiles
+// took 90 and 168 us, with twice the rounding error.
+constexpr int kXc = 16;                        // channels of a split pixel
+constexpr int kInOut = 9 * kCin * kC + kC;     // floats of a block's partial sums
+
+__global__ void __launch_bounds__(256, 2)
+conv_in_wgrad_kernel(const float* __restrict__ f0, const float* __restrict__ f1, const float* __restrict__ f2,
+                     const float* __restrict__ f3, const float* __restrict__ f4, int64_t fb, int64_t fr, int64_t fc,
+                     const bf16* __restrict__ dz, const int32_t* __restrict__ ext, int B, int H, int W, int nstrips,
+                     int nchunk, int rows, int accumulate, float* __restrict__ partials) {
+  constexpr int kXpx = kWgPx + 2;  // pixels x0 - 1 .. x0 + 32
+  constexpr int kStage = (kXpx * kXc + kWgPx * kC);
+  __shared__ __attribute__((aligned(16))) union {
+    bf16 rows[4][kStage];
+    float sums[4][9][8][kC];
+  } sm;
+  const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  bf16* sx = sm.rows[wave];
+  bf16* sz = sx + kXpx * kXc;
+  const uint32_t bytes = (uint32_t)((int64_t)B * H * W * kC * 2);
+  const uint32_t rowbytes = (uint32_t)W * kC * 2;
+  const float* fs[kCin] = {f0, f1, f2, f3, f4};
+
+  f32x4 acc[9][2];
+#pragma unroll
+  for (int t = 0; t < 9; ++t) acc[t][0] = acc[t][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int ntask = B * nstrips * nchunk;
+  for (int task = blockIdx.x * 4 + wave; task < ntask; task += gridDim.x * 4) {
+    const int x0 = (task % nstrips) * kWgPx;
+    const int y0 = ((task / nstrips) % nchunk) * rows;
+    const int b = task / (nstrips * nchunk);
+    int ny, nx;
+    extent_of(ext, b, H, W, ny, nx);
+    const int y1 = min(y0 + rows, ny);
+    if (x0 >= nx || y0 >= y1) continue;
+    const uint32_t img = (uint32_t)b * H * rowbytes;
+    // dz: 16 B of a row per lane, pixel lane / 4 of 16; X: pixel x0 - 1 + lane.
+    // X's addresses are clamped into the extent, its values masked when split.
+    auto off = [&](int x) { return x < nx ? (uint32_t)(x * kC * 2 + (lane & 3) * 16) : kOOB; };
+    const uint32_t oz[2] = {off(x0 + (lane >> 2)), off(x0 + 16 + (lane >> 2))};
+    const int xx = x0 - 1 + lane;
+    const bool okx = (xx >= 0) & (xx < nx);
+    const int64_t ox = (int64_t)b * fb + (int64_t)min(max(xx, 0), nx - 1) * fc;
+    u32x4 stz[kRing][2];
+    float stx[kRing][kCin];
+    // feed j: X row y0 - 1 + j and dz row y0 - 2 + j
+    auto load = [&](int s, int j) {
+      const int yx = y0 - 1 + j, yz = y0 - 2 + j;
+      const bool okz = (yz >= y0) & (yz < y1);
+      const rsrc_t rz = make_rsrc(dz, okz ? bytes : 0u);
+      const uint32_t pz = okz ? img + (uint32_t)yz * rowbytes : 0u;
+      const int64_t oy = (int64_t)min(max(yx, 0), ny - 1) * fr + ox;
+#pragma unroll
+      for (int ci = 0; ci < kCin; ++ci) stx[s][ci] = fs[ci][oy];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) stz[s][i] = __builtin_amdgcn_raw_buffer_load_b128(rz, oz[i], pz, 0);
+    };
+    bf16x8 F[4][3], D[2][2];
+    auto feed = [&](int s, int f, int d, int j) {
+      const int yx = y0 - 1 + j;
+      const bool ok = okx & (yx >= 0) & (yx < ny) & (yx <= y1);
+      uint32_t part[3][kCin];
+#pragma unroll
+      for (int ci = 0; ci < kCin; ++ci) {
+        const float x = ok ? stx[s][ci] : 0.f;
+        part[0][ci] = __float_as_uint(x) & 0xFFFF0000u;
+        const float h = __uint_as_float(part[0][ci]);
+        const float r = x == h ? 0.f : x - h;  // (an infinity has no remainder)
+        part[1][ci] = __float_as_uint(r) & 0xFFFF0000u;
+        part[2][ci] = __float_as_uint(r - __uint_as_float(part[1][ci]));
+      }
+      u32x4 c[2];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t last = i < 3 ? part[i][4] : 0x3F800000u;
+        c[i >> 1][2 * (i & 1)] = (part[0][i] >> 16) | part[1][i];
+        c[i >> 1][2 * (i & 1) + 1] = (part[2][i] >> 16) | (last & 0xFFFF0000u);
+      }
+      if (lane < kXpx) {
+        reinterpret_cast<u32x4*>(sx + lane * kXc)[0] = c[0];
+        reinterpret_cast<u32x4*>(sx + lane * kXc)[1] = c[1];
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) *reinterpret_cast<u32x4*>(sz + i * 16 * kC + lane * 8) = stz[s][i];
+      load(s, j + kRing);
+#pragma unroll
+      for (int t = 0; t < 3; ++t) F[f][t] = transposed<kXc>(sx, t, 0);
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb) D[d][cb] = transposed<kC>(sz, 0, cb);
+    };
+    // products of dz row y0 + j - 3, whose operands feeds j - 3 .. j - 1 read
+    auto mult = [&](int j) {
+#pragma unroll
+      for (int t = 0; t < 9; ++t)
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb)
+          acc[t][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(F[(j + 1 + t / 3) & 3][t % 3], D[(j + 1) & 1][cb],
+                                                               acc[t][cb], 0, 0, 0);
+    };
+#pragma unroll
+    for (int s = 0; s < kRing; ++s) load(s, s);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) feed(j % kRing, j & 3, j & 1, j);
+    const int end = y1 - y0 + 3;
+    for (int j = 3; j < end; j += 4) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        feed((3 + k) % kRing, (3 + k) & 3, (3 + k) & 1, j + k);
+        mult(3 + k);
+      }
+    }
+  }
+
+  // the parts' sums, small ones first, then the four waves' in order
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < 9; ++t)
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb) {
+      const f32x4 a = acc[t][cb];
+      sm.sums[wave][t][g][cb * 16 + n] = (a[2] + a[1]) + a[0];
+      sm.sums[wave][t][4 + g][cb * 16 + n] = a[3];
+    }
+  __syncthreads();
+  float* P = partials + (int64_t)blockIdx.x * kInOut;
+  constexpr int kPer = (kInOut + 255) / 256;
+  float prev[kPer];  // (all loads before the first store)
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    const int i = threadIdx.x + 256 * k;
+    prev[k] = (accumulate && i < kInOut) ? P[i] : 0.f;
+  }
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    const int i = threadIdx.x + 256 * k;
+    if (i >= kInOut) continue;
+    const int co = i % kC, m = i / kC, t = m < 9 * kCin ? m / kCin : 4, ci = m < 9 * kCin ? m % kCin : 7;
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+      v += ci == 4 ? (sm.sums[w][t][6][co] + sm.sums[w][t][5][co]) + sm.sums[w][t][4][co] : sm.sums[w][t][ci][co];
+    P[i] = accumulate ? prev[k] + v : v;
+  }
+}
+
+// Equal shares of the strips' rows for all waves, in multiples of the four
+// steps of the loop; at most 32 rows in a batch of uneven entries, whose
+// padding is skipped.
+inline int strip_rows(const int32_t* ext, int B, int H, int nstrips, int nblocks) {
   const int64_t waves = 4 * (int64_t)nblocks;
-  // Equal shares for all waves, in multiples of the four steps of the loop; at
-  // most 32 rows in a batch of uneven entries, whose padding is skipped.
   int64_t rows = ((int64_t)B * nstrips * H + waves - 1) / waves;
   rows = (rows + 3) / 4 * 4;
-  if (ext && rows > 32) rows = 32;
-  const int nchunk = (int)((H + rows - 1) / rows);
+  return (int)(ext && rows > 32 ? 32 : rows);
+}
+
+int wgrad3x3_launch(const void* act, const void* dz, const int32_t* ext, int B, int H, int W, int nblocks,
+                    float* partials, int accumulate, hipStream_t st) {
+  const int nstrips = (W + kWgPx - 1) / kWgPx, rows = strip_rows(ext, B, H, nstrips, nblocks);
   hipLaunchKernelGGL(wgrad3x3_kernel, dim3(nblocks), dim3(256), 0, st, (const bf16*)act, (const bf16*)dz, ext, B, H, W,
-                     nstrips, nchunk, (int)rows, accumulate, partials);
+                     nstrips, (H + rows - 1) / rows, rows, accumulate, partials);
   IGM_CHECK_LAUNCH();
   return 0;
 }
 
 }  // namespace igm
+
+extern "C" int igm_conv_in_wgrad_partials(const float* f0, const float* f1, const float* f2, const float* f3,
+                                          const float* f4, int64_t fb, int64_t fr, int64_t fc, const int32_t* extents,
+                                          int32_t B, int32_t H, int32_t W, const void* dz1, int32_t nblocks,
+                                          float* partials, int32_t accumulate, void* stream) {
+  using namespace igm;
+  IGM_CHECK_ARG(f0 && f1 && f2 && f3 && f4 && dz1 && partials, "null pointer");
+  IGM_CHECK_ARG(nblocks >= 1 && B >= 1 && H >= 1 && W >= 1, "bad sizes");
+  IGM_CHECK_ARG((int64_t)B * H * W * kC * 2 < (int64_t)kOOB, "activations above 2 GiB (32-bit buffer offsets)");
+  const int nstrips = (W + kWgPx - 1) / kWgPx, rows = strip_rows(extents, B, H, nstrips, nblocks);
+  hipLaunchKernelGGL(conv_in_wgrad_kernel, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, f0, f1, f2, f3, f4, fb, fr,
+                     fc, (const bf16*)dz1, extents, B, H, W, nstrips, (H + rows - 1) / rows, rows, accumulate ? 1 : 0,
+                     partials);
+  IGM_CHECK_LAUNCH();
+  return 0;
+}

@@ -116,3 +116,50 @@ def test_weight_gradient_against_float64(dev, B, H, W, ext, nblocks, accumulate)
         assert float(d) <= 1e-5 * max(float(torch.linalg.vector_norm(ref)), 1.0), (t, float(d))
     ref = zm.sum(0) + accumulate
     assert float(torch.linalg.vector_norm(db.double() - ref)) <= 1e-5 * max(float(torch.linalg.vector_norm(ref)), 1.0)
+
+
+@pytest.mark.parametrize("nblocks,accumulate", [(1, 0), (3, 1), (512, 0)])
+@pytest.mark.parametrize("layout", ["planar", "nhwc", "transposed"])
+@pytest.mark.parametrize("B,H,W,ext", [(1, 1, 1, None), (2, 13, 64, [(13, 31), (7, 64)]),
+                                       (3, 66, 70, [(65, 70), (66, 5), (1, 1)]), (1, 300, 257, None)])
+def test_layer1_weight_gradient_against_float64(dev, B, H, W, ext, layout, nblocks, accumulate):
+    """igm_conv_in_wgrad on raw magnitudes for every layout of the fields; the
+    tolerance is the 3x3 layers' (the same chains), per field."""
+    gen = torch.Generator().manual_seed(H * W)
+    scale = torch.tensor([800.0, 3000.0, 100.0, 0.05, 100.0])
+    X = (torch.rand((B, H, W, 5), generator=gen) * scale).to(dev)
+    dz = torch.randn((B, H, W, 32), generator=gen).to(torch.bfloat16).to(dev)
+    if layout == "nhwc":
+        fs, strides = [X[..., i] for i in range(5)], (H * W * 5, W * 5, 5)
+    elif layout == "planar":
+        fs, strides = [X[..., i].contiguous() for i in range(5)], (H * W, W, 1)
+    else:
+        fs, strides = [X[..., i].transpose(1, 2).contiguous() for i in range(5)], (H * W, 1, H)
+    e = None if ext is None else torch.tensor(ext, dtype=torch.int32, device=dev)
+    ws = torch.full((L.load().igm_wgrad_workspace_floats(0, nblocks),), float("nan"), device=dev)
+    dW, db = torch.ones((3, 3, 5, 32), device=dev), torch.ones(32, device=dev)
+    L.call("igm_conv_in_wgrad", *[L.ptr(f) for f in fs], *strides, L.ptr(e), B, H, W, L.ptr(dz), nblocks, L.ptr(ws),
+           accumulate, L.ptr(dW), L.ptr(db), L.stream_ptr())
+    torch.cuda.synchronize()
+    xp = torch.nn.functional.pad(masked(X, ext).double(), (0, 0, 1, 1, 1, 1))
+    zm = masked(dz, ext).double().reshape(-1, 32)
+    ref = torch.stack([xp[:, t // 3:t // 3 + H, t % 3:t % 3 + W].reshape(-1, 5).t().contiguous() @ zm for t in range(9)])
+    d = (dW.reshape(9, 5, 32).double() - ref - accumulate).transpose(0, 1).reshape(5, -1)
+    n = ref.transpose(0, 1).reshape(5, -1)
+    assert (d.norm(dim=1) <= 1e-5 * n.norm(dim=1).clamp(min=1.0)).all(), d.norm(dim=1) / n.norm(dim=1)
+    rb = zm.sum(0) + accumulate
+    assert float((db.double() - rb).norm()) <= 1e-5 * max(float(rb.norm()), 1.0)
+
+
+def test_layer1_weight_gradient_of_an_infinite_input(dev):
+    """An infinity or NaN among the inputs reaches the entries it multiplies,
+    as a float32 product would carry it, and no others."""
+    X = torch.ones((1, 8, 8, 5), device=dev)
+    X[0, 4, 4, 1], X[0, 2, 6, 3] = float("inf"), float("nan")
+    dz = torch.ones((1, 8, 8, 32), dtype=torch.bfloat16, device=dev)
+    ws = torch.empty(L.load().igm_wgrad_workspace_floats(0, 4), device=dev)
+    dW, db = torch.empty((3, 3, 5, 32), device=dev), torch.empty(32, device=dev)
+    L.call("igm_conv_in_wgrad", *[X.data_ptr() + 4 * i for i in range(5)], 320, 40, 5, None, 1, 8, 8, L.ptr(dz), 4,
+           L.ptr(ws), 0, L.ptr(dW), L.ptr(db), L.stream_ptr())
+    assert torch.isposinf(dW[:, :, 1]).all() and torch.isnan(dW[:, :, 3]).all()
+    assert torch.isfinite(dW[:, :, [0, 2, 4]]).all() and torch.isfinite(db).all()
