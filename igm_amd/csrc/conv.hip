@@ -8,9 +8,7 @@
 // makes a padded batch behave exactly like per-entry "same" zero padding.
 //
 // Kernels:
-//  conv_in_kernel       layer 1 (5 -> 32), fp32 VALU (raw inputs such as the
-//                       surface elevation need fp32: bf16 spacing is 16 m at
-//                       2500-3000 m), bias + LeakyReLU, bf16 out.
+//  (layer 1: conv_in.hip)
 //  (the 32 -> 32 3x3 layers, forward and data gradient: conv3x3.hip)
 //  head_mfma_kernel     1x1 32 -> 2Nz (<= 32) output layer, fp32 out.
 //  wgrad1x1_kernel      weight gradient of the head: K = pixels; tiles are
@@ -29,62 +27,8 @@ namespace igm {
 constexpr int kTileW = 64;    // pixels per tile row
 constexpr int kChStride = 72; // LDS channel-row stride in bf16 (144 B) for wgrad
 
-// ------------------------------------------------------------ layer 1 --
-// One thread per output pixel.  The 45 inputs of its 3x3 window are loaded
-// up front; the weights (HWIO [3][3][5][32] fp32) are wave-uniform, so they
-// come through scalar loads (read-only, no LDS) as the FMA operand.  Each
-// output channel accumulates bias, then taps 0..8, then fields 0..4.
-__global__ void __launch_bounds__(256)
-conv_in_kernel(const float* __restrict__ f0, const float* __restrict__ f1,
-               const float* __restrict__ f2, const float* __restrict__ f3,
-               const float* __restrict__ f4, int64_t fb, int64_t fr, int64_t fc,
-               const int32_t* __restrict__ ext, int H, int W, const float* __restrict__ w,
-               const float* __restrict__ bias, bf16* __restrict__ out) {
-  const int x = blockIdx.x * blockDim.x + threadIdx.x;
-  const int y = blockIdx.y;
-  const int b = blockIdx.z;
-  if (x >= W) return;
-  int ny, nx;
-  extent_of(ext, b, H, W, ny, nx);
-  bf16* o = out + (((int64_t)b * H + y) * W + x) * kC;
-  if (y >= ny || x >= nx) {
-    uint4 z = {0, 0, 0, 0};
-#pragma unroll
-    for (int q = 0; q < 4; ++q) reinterpret_cast<uint4*>(o)[q] = z;
-    return;
-  }
-  const float* fs[kCin] = {f0, f1, f2, f3, f4};
-  float v[9][kCin];
-#pragma unroll
-  for (int t = 0; t < 9; ++t) {
-    const int yy = y + t / 3 - 1, xx = x + t % 3 - 1;
-    const bool in = yy >= 0 && yy < ny && xx >= 0 && xx < nx;
-    const int64_t off = (int64_t)b * fb + (int64_t)yy * fr + (int64_t)xx * fc;
-#pragma unroll
-    for (int ci = 0; ci < kCin; ++ci) v[t][ci] = in ? fs[ci][off] : 0.f;
-  }
-  float acc[kC];
-#pragma unroll
-  for (int c = 0; c < kC; ++c) acc[c] = bias[c];
-#pragma unroll
-  for (int t = 0; t < 9; ++t)
-#pragma unroll
-    for (int ci = 0; ci < kCin; ++ci) {
-      const float* wr = w + (t * kCin + ci) * kC;
-#pragma unroll
-      for (int c = 0; c < kC; ++c) acc[c] += v[t][ci] * wr[c];
-    }
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    bf16x8 h;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) h[e] = f2bf(leaky(acc[q * 8 + e]));
-    reinterpret_cast<bf16x8*>(o)[q] = h;
-  }
-}
-
 // Gradient of the network with respect to its 5 input fields, through
-// layer 1: the transpose of conv_in_kernel's cross-correlation,
+// layer 1: the transpose of its cross-correlation,
 //   dX[b, y, x, ci] = sum_{r, s, co} W[r][s][ci][co] * dz1[b, y - r + 1, x - s + 1, co],
 // zero padding, fp32 accumulation in a fixed order; dz1 (bf16 NHWC, 32
 // channels) is the gradient at layer 1's pre-activation output.  Zeros
@@ -652,19 +596,6 @@ inline int grid_for(int64_t n, int b = 256) { return (int)((n + b - 1) / b); }
 using namespace igm;
 
 extern "C" {
-
-int igm_conv_in_fwd(const float* f0, const float* f1, const float* f2, const float* f3,
-                    const float* f4, int64_t fb, int64_t fr, int64_t fc, const int32_t* extents,
-                    int32_t B, int32_t H, int32_t W, const float* w_hwio, const float* bias,
-                    void* out_bf16, void* stream) {
-  IGM_CHECK_ARG(f0 && f1 && f2 && f3 && f4 && w_hwio && bias && out_bf16, "null pointer");
-  IGM_CHECK_ARG(B >= 1 && H >= 1 && W >= 1 && H <= 65535 && B <= 65535, "bad sizes");
-  hipLaunchKernelGGL(conv_in_kernel, dim3(grid_for(W), H, B), dim3(256), 0, (hipStream_t)stream,
-                     f0, f1, f2, f3, f4, fb, fr, fc, extents, H, W, w_hwio, bias,
-                     (bf16*)out_bf16);
-  IGM_CHECK_LAUNCH();
-  return 0;
-}
 
 int igm_conv1x1_head_fwd(const void* in, const void* wpacked, const float* bias,
                          const int32_t* extents, int32_t B, int32_t H, int32_t W, int32_t cout,

@@ -163,3 +163,49 @@ def test_layer1_weight_gradient_of_an_infinite_input(dev):
            L.ptr(ws), 0, L.ptr(dW), L.ptr(db), L.stream_ptr())
     assert torch.isposinf(dW[:, :, 1]).all() and torch.isnan(dW[:, :, 3]).all()
     assert torch.isfinite(dW[:, :, [0, 2, 4]]).all() and torch.isfinite(db).all()
+
+
+@pytest.mark.parametrize("layout", ["planar", "nhwc", "transposed"])
+@pytest.mark.parametrize("B,H,W,ext", [(1, 1, 1, None), (1, 2, 63, None), (1, 5, 64, None), (1, 3, 65, None),
+                                       (3, 66, 70, [(65, 70), (66, 5), (1, 1)]), (2, 300, 130, [(300, 128), (7, 64)]),
+                                       (1, 700, 600, None)])
+def test_layer1_against_float64(dev, B, H, W, ext, layout):
+    """igm_conv_in_fwd element by element: half a bf16 step of the result, and
+    the float32 rounding of a chain of 45 FMAs, at most 46 * 2^-24 * (|b| + sum
+    |w x|) (2^-8 and 3e-6 of it are asked); zeros outside the extents."""
+    gen = torch.Generator().manual_seed(H * W)
+    X = (torch.rand((B, H, W, 5), generator=gen) * torch.tensor([800.0, 3000.0, 100.0, 0.05, 100.0])).to(dev)
+    w, b = torch.randn((9, 5, 32), generator=gen).to(dev), torch.randn(32, generator=gen).to(dev)
+    if layout == "nhwc":
+        fs, strides = [X[..., i] for i in range(5)], (H * W * 5, W * 5, 5)
+    elif layout == "planar":
+        fs, strides = [X[..., i].contiguous() for i in range(5)], (H * W, W, 1)
+    else:
+        fs, strides = [X[..., i].transpose(1, 2).contiguous() for i in range(5)], (H * W, 1, H)
+    e = None if ext is None else torch.tensor(ext, dtype=torch.int32, device=dev)
+    out = torch.full((B, H, W, 32), float("nan"), dtype=torch.bfloat16, device=dev)
+    L.call("igm_conv_in_fwd", *[L.ptr(f) for f in fs], *strides, L.ptr(e), B, H, W, L.ptr(w), L.ptr(b), L.ptr(out),
+           L.stream_ptr())
+    torch.cuda.synchronize()
+    xp = torch.nn.functional.pad(masked(X, ext).double(), (0, 0, 1, 1, 1, 1))
+    ref = b.double().expand(B, H, W, 32).clone()
+    mag = ref.abs()
+    for t in range(9):
+        part = xp[:, t // 3:t // 3 + H, t % 3:t % 3 + W].reshape(-1, 5)
+        ref += (part @ w[t].double()).view(B, H, W, 32)
+        mag += (part.abs() @ w[t].double().abs()).view(B, H, W, 32)
+    ref = masked(torch.where(ref > 0, ref, 0.01 * ref), ext)
+    assert ((out.double() - ref).abs() <= 2.0**-8 * ref.abs() + masked(3e-6 * mag, ext)).all()
+
+
+def test_layer1_of_an_infinite_input(dev):
+    """An infinity reaches the 3x3 pixels around it and no others."""
+    X = torch.ones((1, 9, 80, 5), device=dev)
+    X[0, 4, 70, 1] = float("inf")
+    w, b = torch.ones((9, 5, 32), device=dev), torch.zeros(32, device=dev)
+    out = torch.zeros((1, 9, 80, 32), dtype=torch.bfloat16, device=dev)
+    L.call("igm_conv_in_fwd", *[X.data_ptr() + 4 * i for i in range(5)], 3600, 400, 5, None, 1, 9, 80, L.ptr(w),
+           L.ptr(b), L.ptr(out), L.stream_ptr())
+    near = torch.zeros((9, 80), dtype=torch.bool, device=dev)
+    near[3:6, 69:72] = True
+    assert torch.isposinf(out[0, near]).all() and torch.isfinite(out[0, ~near]).all()
