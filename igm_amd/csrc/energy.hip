@@ -21,7 +21,7 @@
 // gradient is a deterministic gather.
 //
 // Per-cell coefficients that do not depend on (U, V) are computed once per
-// solve by energy_coeffs_kernel (7 planes, 28 B per cell).
+// solve (7 planes, 28 B per cell: energy_coeffs.hip).
 #include "energy_pass.hpp"
 
 #include <mutex>
@@ -36,79 +36,6 @@ thread_local std::string g_last_error;
 }
 void set_error(const std::string& msg) { g_last_error = msg; }
 const char* last_error() { return g_last_error.c_str(); }
-
-// --------------------------------------------------------- coefficients --
-//
-// Plane meaning for the cell with lower-left node (j, i) (S = number of cells):
-//   0  q  = dx * damp / max(H, thr)        damp = 1, or 0.01 where stag4h(C) <= 0
-//   1  w  = H * Bs / (p * S)               Bs = stag4h(2 A^(-1/n)), p = 1 + 1/n
-//   2  gx = 0.25 * rho*g*1e-6 * H * sx / S (sx, sy: staggered slope of usurf)
-//   3  gy = 0.25 * rho*g*1e-6 * H * sy / S
-//   4  cs = stag4h(C) / (s * S)            s = 1 + 1/m
-//   5  bx, 6 by: staggered slope of the bed usurf - thk
-// The 0.25 factors absorb the 1/4 of the horizontal node average, which the
-// pass keeps unscaled (sum of the 4 corner nodes); dx in q puts the vertical
-// derivative in the pass's units of 1/(4 dx) (dx = dX[b, 0, 0], the scalar
-// spacing of the velocity derivatives, cost_shear.py:113).
-template <typename T>
-__global__ void __launch_bounds__(256)
-energy_coeffs_kernel(const T* __restrict__ thk, const T* __restrict__ usurf,
-                     const T* __restrict__ arrh, const T* __restrict__ slid,
-                     const T* __restrict__ dX, int64_t fb, int64_t fr, int64_t fc,
-                     const int32_t* __restrict__ extents, int Ny, int Nx, T inv_n, T inv_p,
-                     T inv_s, T thr, T rho_g, T* __restrict__ coef, T* __restrict__ hscale) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int j = blockIdx.y;
-  const int b = blockIdx.z;
-  if (i >= Nx) return;
-  const int ny = extents ? min(extents[2 * b], Ny) : Ny;
-  const int nx = extents ? min(extents[2 * b + 1], Nx) : Nx;
-  const int64_t plane = (int64_t)Ny * Nx;
-  T* cb = coef + (int64_t)b * kPlanes * plane + (int64_t)j * Nx + i;
-  const int64_t base = (int64_t)b * fb;
-  if (i == 0 && j == 0) hscale[b] = T(1) / (T(4) * dX[base]);
-  if (!(j < ny - 1 && i < nx - 1)) {
-#pragma unroll
-    for (int p = 0; p < kPlanes; ++p) cb[p * plane] = T(0);
-    return;
-  }
-  const int64_t o00 = base + (int64_t)j * fr + (int64_t)i * fc;
-  const int64_t o01 = o00 + fc;       // (j, i+1)
-  const int64_t o10 = o00 + fr;       // (j+1, i)
-  const int64_t o11 = o00 + fr + fc;  // (j+1, i+1)
-  auto st4 = [](T a11, T a10, T a01, T a00) { return (a11 + a10 + a01 + a00) / T(4); };
-  const T t00 = thk[o00], t01 = thk[o01], t10 = thk[o10], t11 = thk[o11];
-  const T s00 = usurf[o00], s01 = usurf[o01], s10 = usurf[o10], s11 = usurf[o11];
-  const T d00 = dX[o00], d01 = dX[o01], d10 = dX[o10], d11 = dX[o11];
-  const T H = st4(t11, t10, t01, t00);
-  const T Bs = st4(T(2) * pow(arrh[o11], -inv_n), T(2) * pow(arrh[o10], -inv_n),
-                   T(2) * pow(arrh[o01], -inv_n), T(2) * pow(arrh[o00], -inv_n));
-  const T Cs = st4(slid[o11], slid[o10], slid[o01], slid[o00]);
-  // compute_gradient.py:10-14 on s = usurf (surface) and s = usurf - thk (bed)
-  auto gx = [&](T a00, T a01, T a10, T a11) {
-    const T e0 = T(2) * (a01 - a00) / (d01 + d00);
-    const T e1 = T(2) * (a11 - a10) / (d11 + d10);
-    return T(0.5) * (e1 + e0);
-  };
-  auto gy = [&](T a00, T a01, T a10, T a11) {
-    const T e0 = T(2) * (a10 - a00) / (d10 + d00);
-    const T e1 = T(2) * (a11 - a01) / (d11 + d01);
-    return T(0.5) * (e1 + e0);
-  };
-  const T sx = gx(s00, s01, s10, s11), sy = gy(s00, s01, s10, s11);
-  const T b00 = s00 - t00, b01 = s01 - t01, b10 = s10 - t10, b11 = s11 - t11;
-  const T bx = gx(b00, b01, b10, b11), by = gy(b00, b01, b10, b11);
-  const T inv_S = T(1) / (T(ny - 1) * T(nx - 1));
-  const T damp = Cs > T(0) ? T(1) : T(0.01);
-  const T Hc = H > thr ? H : thr;
-  cb[0 * plane] = dX[base] * damp / Hc;
-  cb[1 * plane] = H * Bs * inv_p * inv_S;
-  cb[2 * plane] = T(0.25) * rho_g * H * sx * inv_S;
-  cb[3 * plane] = T(0.25) * rho_g * H * sy * inv_S;
-  cb[4 * plane] = Cs * inv_s * inv_S;
-  cb[5 * plane] = bx;
-  cb[6 * plane] = by;
-}
 
 // ------------------------------------------------------------- finalize --
 //
@@ -389,27 +316,6 @@ struct VwArr {
 
 // ------------------------------------------------------------- dispatch --
 
-template <typename T>
-int coeffs_impl(const T* thk, const T* usurf, const T* arrh, const T* slid, const T* dX,
-                int64_t fb, int64_t fr, int64_t fc, const int32_t* extents, int nbatch, int Ny,
-                int Nx, const IgmPhysics* phys, T* coef, T* hscale, void* stream) {
-  IGM_CHECK_ARG(thk && usurf && arrh && slid && dX && coef && hscale && phys, "null pointer");
-  IGM_CHECK_ARG(nbatch >= 1 && Ny >= 2 && Nx >= 2, "need nbatch >= 1 and a grid of at least 2 x 2");
-  IGM_CHECK_ARG(Ny <= 65535, "Ny must be <= 65535");
-  IGM_CHECK_ARG(phys->force_negative_gravitational_energy == 0,
-                "force_negative_gravitational_energy is not supported");
-  const T inv_n = T(1.0 / phys->exp_glen);
-  const T p = T(1.0 + 1.0 / phys->exp_glen);
-  const T s = T(1.0 + 1.0 / phys->exp_weertman);
-  const T rho_g = T(phys->ice_density * phys->gravity_cst * 1e-6);
-  dim3 grid((Nx + 255) / 256, Ny, nbatch);
-  hipLaunchKernelGGL(energy_coeffs_kernel<T>, grid, dim3(256), 0, (hipStream_t)stream, thk,
-                     usurf, arrh, slid, dX, fb, fr, fc, extents, Ny, Nx, inv_n, T(1) / p, T(1) / s,
-                     T(phys->thr_ice_thk), rho_g, coef, hscale);
-  IGM_CHECK_LAUNCH();
-  return 0;
-}
-
 template <typename T, int MODE, int INTER>
 void launch_pass_nz(int nz, dim3 grid, hipStream_t st, const PassArgs<T>& a, bool* ok) {
   *ok = true;
@@ -663,23 +569,6 @@ int64_t igm_energy_workspace_doubles(int32_t nbatch, int32_t Ny, int32_t Nx) {
   const igm::PassGeom g2 = igm::pair_pass_geom(Ny, Nx);
   const int64_t one = 3 * (int64_t)nbatch * g.blocks, two = 6 * (int64_t)g2.blocks;
   return one > two ? one : two;
-}
-
-int igm_energy_coeffs_f32(const float* thk, const float* usurf, const float* arrhenius,
-                          const float* slidingco, const float* dX, int64_t fb, int64_t fr,
-                          int64_t fc, const int32_t* extents, int32_t nbatch, int32_t Ny,
-                          int32_t Nx, const IgmPhysics* phys, float* coef, float* hscale,
-                          void* stream) {
-  return igm::coeffs_impl<float>(thk, usurf, arrhenius, slidingco, dX, fb, fr, fc, extents, nbatch,
-                                 Ny, Nx, phys, coef, hscale, stream);
-}
-int igm_energy_coeffs_f64(const double* thk, const double* usurf, const double* arrhenius,
-                          const double* slidingco, const double* dX, int64_t fb, int64_t fr,
-                          int64_t fc, const int32_t* extents, int32_t nbatch, int32_t Ny,
-                          int32_t Nx, const IgmPhysics* phys, double* coef, double* hscale,
-                          void* stream) {
-  return igm::coeffs_impl<double>(thk, usurf, arrhenius, slidingco, dX, fb, fr, fc, extents,
-                                  nbatch, Ny, Nx, phys, coef, hscale, stream);
 }
 
 int igm_energy_pass_f32(int32_t mode, int32_t nz, int32_t nbatch, int32_t Ny, int32_t Nx,
