@@ -252,7 +252,9 @@ struct CellEnergy {
 // NZ-1 in order, then finish().  level(k) emits level k-1 (k >= 1) and
 // finish() emits level NZ-1, so a caller can interleave two sweeps whose
 // inputs depend on each other's outputs (the two-iteration pass).
-template <typename T, int NZ>
+//
+// THIRD (float64): both powers are within 1e-12 of -1/3 (pow_third).
+template <typename T, int NZ, bool THIRD = false>
 struct LevelSweep {
   const PassArgs<T>& a;
   const T hh2, h05, h025;
@@ -310,7 +312,9 @@ struct LevelSweep {
       const T ub = T(0.25) * sU, vb = T(0.25) * sV;
       const T c2 = ub * bx + vb * by;
       const T N = (ub * ub + vb * vb) + a.regu_w2 + c2 * c2;
-      const T t = pow_pos(N, a.e_slid);  // N^(s/2 - 1)
+      T t;  // N^(s/2 - 1)
+      if constexpr (THIRD) t = pow_third(N, a.e_slid);
+      else t = pow_pos(N, a.e_slid);
       c_sl = csl * N * t;
       const T gs = T(0.25) * csl * a.s_slid * t;
       n_su += gs * (ub + c2 * bx);
@@ -333,7 +337,9 @@ struct LevelSweep {
       const T sclip = clamp_(sr2, a.min_sr2, a.max_sr2);
       const bool in_rng = (sclip == sr2);  // the clip passes its gradient inside the range
       const T sc = sclip + a.regu2;
-      const T wl = scaled_pow(sc, a.e_glen, a.dz[l], a.l2dz[l]);  // dzeta_l sc^e
+      T wl;  // dzeta_l sc^e
+      if constexpr (THIRD) wl = a.dz[l] * pow_third(sc, a.e_glen);
+      else wl = scaled_pow(sc, a.e_glen, a.dz[l], a.l2dz[l]);
       c_sh += wl * sr2;
       // adjoint of the layer (in the scaled variables):
       // G = w hh2 wl (1 + e sr2 / sc), zero ratio outside the clip range
@@ -372,13 +378,13 @@ struct LevelSweep {
   }
 };
 
-template <typename T, int NZ, typename Emit>
+template <typename T, int NZ, bool THIRD, typename Emit>
 __device__ __forceinline__ CellEnergy<T> level_sweep(const PassArgs<T>& a, T hh2, T h05, T h025,
                                                     const T (&up)[NZ], const T (&vp)[NZ],
                                                     const T (&uc)[NZ], const T (&vc)[NZ],
                                                     const T (&cc)[kPlanes], T (&cu)[NZ],
                                                     T (&cv)[NZ], Emit&& emit) {
-  LevelSweep<T, NZ> sw(a, hh2, h05, h025, cc);
+  LevelSweep<T, NZ, THIRD> sw(a, hh2, h05, h025, cc);
 #pragma unroll
   for (int k = 0; k < NZ; ++k) sw.level(k, up[k], vp[k], uc[k], vc[k], cu, cv, emit);
   return sw.finish(cu, cv, emit);
