@@ -28,9 +28,6 @@ namespace igm {
 constexpr int kStripPx = 64;            // pixels of a wave's row
 constexpr int kPairPx = kStripPx - 2;   // columns a wave of the two-layer kernel owns
 
-// cache policy of a kernel's stores: cached, non-temporal, written through
-constexpr int kStoreCached = 0, kStoreStream = 2, kStoreThrough = 16;
-
 struct ConvGeom {
   int nstrips, nrowblk, rows, blocks;
 };
@@ -103,7 +100,7 @@ __device__ __forceinline__ ConvTile conv_tile(const ConvArgs& a, int own) {
   return t;
 }
 __device__ __forceinline__ const u32x4* weight_frag(const bf16* wt, const ConvTile& t, int tap, int cb) {
-  return reinterpret_cast<const u32x4*>(wt + ((tap * kC + 8 * (t.n >> 2) + 4 * cb + (t.n & 3)) * kC + 8 * t.g));
+  return conv_weight_frag(wt, t.n, t.g, tap, cb);
 }
 // A row's 16 B per lane to byte offset off (kOOB: dropped) of the row at so.
 // The row's offset is added to the lane's, not given in the instruction's
@@ -389,18 +386,6 @@ ConvArgs conv_args(const void* in, const void* w, const float* bias, const void*
   return a;
 }
 int64_t act_bytes(int B, int H, int W) { return (int64_t)B * H * W * kC * 2; }
-// How a layer's output of so many bytes is stored.  The caches write it back
-// at the kernel's end otherwise: written through, 500 x 500 takes 8.6 us
-// instead of 10.5 and 1000 x 1000 (64 MB) 22.7 instead of 24.0.  Buffers that
-// do not stay in the 256 MB last-level cache together gain nothing from it:
-// 1500 x 1500 (144 MB, forward) took 59 to 61 us either way, and the data
-// gradient, which also reads the activation, 75.7 us with non-temporal
-// stores, 88 without (8 x 512 x 512, 134 MB: 63.9 and 71.9).  The forward
-// pass of such a batch keeps them cached (41 us, 50 non-temporal).
-inline int store_mode(int64_t bytes, bool dgrad) {
-  if (bytes <= (80 << 20)) return kStoreThrough;
-  return dgrad && bytes >= (120 << 20) ? kStoreStream : kStoreCached;
-}
 }  // namespace
 
 extern "C" {
@@ -415,7 +400,7 @@ int igm_conv3x3_fwd_bf16(const void* in, const void* wpacked, const float* bias,
   const ConvArgs a = conv_args(in, wpacked, bias, nullptr, extents, B, H, W, out, kStripPx);
   const dim3 grid(a.g.blocks), block(256);
   hipStream_t st = (hipStream_t)stream;
-  switch (store_mode(act_bytes(B, H, W), false)) {
+  switch (conv_store_mode(act_bytes(B, H, W), false)) {
     case kStoreThrough: hipLaunchKernelGGL((conv3x3_kernel<0, kStoreThrough>), grid, block, 0, st, a); break;
     default: hipLaunchKernelGGL((conv3x3_kernel<0, kStoreCached>), grid, block, 0, st, a); break;
   }
@@ -435,7 +420,7 @@ int igm_conv3x3_pair_fwd_bf16(const void* in, const void* w1, const float* b1, c
   a.bias[1] = b2;
   const dim3 grid(a.g.blocks), block(256);
   hipStream_t st = (hipStream_t)stream;
-  switch (store_mode(act_bytes(B, H, W), false)) {
+  switch (conv_store_mode(act_bytes(B, H, W), false)) {
     case kStoreThrough: hipLaunchKernelGGL((conv3x3_pair_kernel<kStoreThrough>), grid, block, 0, st, a); break;
     default: hipLaunchKernelGGL((conv3x3_pair_kernel<kStoreCached>), grid, block, 0, st, a); break;
   }
@@ -453,7 +438,7 @@ int igm_conv3x3_dgrad_bf16(const void* dz, const void* wpacked_dgrad, const void
   const ConvArgs a = conv_args(dz, wpacked_dgrad, nullptr, act_below, extents, B, H, W, dz_below, kStripPx);
   const dim3 grid(a.g.blocks), block(256);
   hipStream_t st = (hipStream_t)stream;
-  switch (store_mode(act_bytes(B, H, W), true)) {
+  switch (conv_store_mode(act_bytes(B, H, W), true)) {
     case kStoreThrough: hipLaunchKernelGGL((conv3x3_kernel<1, kStoreThrough>), grid, block, 0, st, a); break;
     case kStoreStream: hipLaunchKernelGGL((conv3x3_kernel<1, kStoreStream>), grid, block, 0, st, a); break;
     default: hipLaunchKernelGGL((conv3x3_kernel<1, kStoreCached>), grid, block, 0, st, a); break;

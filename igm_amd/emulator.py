@@ -153,25 +153,19 @@ class CNN:
         st = L.stream_ptr()
         # deferred: the sub-batches add up in the partial sums; otherwise this
         # batch's are summed (into self.g, added when accumulate) at the end
-        part, nb = self._deferred_partials(nblocks) if deferred else self._partials(nblocks)
+        part, nb = self._deferred_partials(nblocks) if deferred else self._partials(nblocks, (B, H, W))
         acc = 1 if accumulate and deferred else 0
-
-        def wgrad(li, taps, a, d):
-            L.call("igm_conv_wgrad_partials_bf16", taps, L.ptr(a), L.ptr(d), ext, B, H, W, nb[taps],
-                   L.ptr(part[li]), acc, st)
-
         nl = self.nl
         dz = torch.empty((B, H, W, NF), dtype=torch.bfloat16, device=self.device)
         dYb = torch.empty_like(dz)
         L.call("igm_conv1x1_head_bwd", L.ptr(dY), L.ptr(acts[nl - 1]), L.ptr(self.kernel(nl)), ext, B, H,
                W, self.cout, L.ptr(dz), L.ptr(dYb), st)
-        wgrad(nl, 1, acts[nl - 1], dYb)
+        L.call("igm_conv_wgrad_partials_bf16", 1, L.ptr(acts[nl - 1]), L.ptr(dYb), ext, B, H, W, nb[1],
+               L.ptr(part[nl]), acc, st)
         below = dYb  # reuse as the ping-pong buffer
         for li in range(nl - 1, 0, -1):  # layer index li (0-based) is a 3x3 MFMA layer
-            a_in = acts[li - 1]
-            wgrad(li, 9, a_in, dz)
-            L.call("igm_conv3x3_dgrad_bf16", L.ptr(dz), L.ptr(self.dgr[li - 1]), L.ptr(a_in), ext, B, H,
-                   W, L.ptr(below), st)
+            L.call("igm_conv3x3_bwd_bf16", L.ptr(acts[li - 1]), L.ptr(dz), L.ptr(self.dgr[li - 1]), ext, B, H, W,
+                   nb[9], L.ptr(part[li]), acc, L.ptr(below), st)
             dz, below = below, dz
         L.call("igm_conv_in_wgrad_partials", *fptrs, fb, fr, fc, ext, B, H, W, L.ptr(dz), nb[0], L.ptr(part[0]),
                acc, st)
@@ -183,18 +177,25 @@ class CNN:
             L.call("igm_conv_in_dgrad", L.ptr(dz), L.ptr(self.kernel(0)), ext, B, H, W, L.ptr(input_grad), st)
         return self.g
 
-    # The 3x3 layers' weight gradient runs one wave per SIMD, 256 blocks at
-    # once; more partial-sum rows would only take more rounds (1000 x 1000:
-    # 25.5 us a layer with 256 rows, 32.6 with 512).
+    # The 3x3 layers' backward kernel runs one wave per SIMD, 256 blocks at
+    # once; more partial-sum rows would only take more rounds.
     WGRAD_BLOCKS = 256
 
-    def _partials(self, nblocks):
+    def _partials(self, nblocks, size=None):
         """Partial-sum buffers of every layer (layer 0: layer 1's layout;
         1..nl-1: 3x3, one after the other; nl: the 1x1 head) and their rows by
-        kind (0, 9 taps, 1 tap)."""
+        kind (0, 9 taps, 1 tap).  ``size`` (B, H, W): no more rows than there
+        are blocks with work, four pieces of 4 rows x 32 columns each (the head:
+        one of 4 x 64); at 256 x 319 the reduction takes 27 us without."""
         lib = L.load()
         nb = {0: nblocks, 9: min(nblocks, self.WGRAD_BLOCKS), 1: nblocks}
+        if size is not None:
+            B, H, W = size
+            quads = B * ((H + 3) // 4)
+            work = {0: (quads * ((W + 31) // 32) + 3) // 4, 1: quads * ((W + 63) // 64)}
+            nb = {t: min(nb[t], work[1 if t == 1 else 0]) for t in nb}
         n = {t: lib.igm_wgrad_workspace_floats(t, nb[t]) for t in nb}
+        # (each part a multiple of 16 B)
         flat = torch.empty(n[0] + (self.nl - 1) * n[9] + n[1], dtype=torch.float32, device=self.device)
         return flat.split([n[0]] + [n[9]] * (self.nl - 1) + [n[1]]), nb
 

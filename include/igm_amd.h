@@ -325,6 +325,11 @@ int igm_conv_wgrad_partials_bf16(int32_t taps, const void* act, const void* dz,
                                  const int32_t* extents, int32_t B, int32_t H, int32_t W,
                                  int32_t nblocks, float* partials, int32_t accumulate,
                                  void* stream);
+/* igm_conv_wgrad_partials_bf16 (taps 9) of a layer and the igm_conv3x3_dgrad_bf16
+ * below it in one pass over dz and act, bit for bit what the two calls give. */
+int igm_conv3x3_bwd_bf16(const void* act, const void* dz, const void* wpacked_dgrad,
+                         const int32_t* extents, int32_t B, int32_t H, int32_t W, int32_t nblocks,
+                         float* partials, int32_t accumulate, void* dz_below, void* stream);
 int igm_conv_in_wgrad_partials(const float* f0, const float* f1, const float* f2, const float* f3,
                                const float* f4, int64_t fb, int64_t fr, int64_t fc,
                                const int32_t* extents, int32_t B, int32_t H, int32_t W,

@@ -209,3 +209,61 @@ def test_layer1_of_an_infinite_input(dev):
     near = torch.zeros((9, 80), dtype=torch.bool, device=dev)
     near[3:6, 69:72] = True
     assert torch.isposinf(out[0, near]).all() and torch.isfinite(out[0, ~near]).all()
+
+
+@pytest.mark.parametrize("nblocks,accumulate", [(1, 0), (3, 1), (256, 0), (300, 1)])
+@pytest.mark.parametrize("B,H,W,ext", [(1, 1, 1, None), (1, 5, 33, None), (1, 64, 32, None),
+                                       (2, 13, 64, [(13, 31), (7, 64)]), (3, 66, 70, [(65, 70), (66, 5), (1, 1)]),
+                                       (1, 300, 257, None), (2, 700, 600, [(700, 600), (31, 599)])])
+def test_backward_in_one_pass_equals_two(dev, B, H, W, ext, nblocks, accumulate):
+    """igm_conv3x3_bwd_bf16 runs the products of igm_conv_wgrad_partials_bf16
+    and igm_conv3x3_dgrad_bf16 in their order: equal bits."""
+    act, (w, _), _ = case(B, H, W, dev)
+    dz = torch.randn((B, H, W, 32), generator=torch.Generator().manual_seed(H)).to(torch.bfloat16).to(dev)
+    e = None if ext is None else torch.tensor(ext, dtype=torch.int32, device=dev)
+    n, st = L.load().igm_wgrad_workspace_floats(9, nblocks), L.stream_ptr()
+    p1, p2 = torch.ones(n, device=dev), torch.ones(n, device=dev)
+    o1, o2 = torch.full_like(act, float("nan")), torch.full_like(act, float("nan"))
+    L.call("igm_conv_wgrad_partials_bf16", 9, L.ptr(act), L.ptr(dz), L.ptr(e), B, H, W, nblocks, L.ptr(p1), accumulate,
+           st)
+    L.call("igm_conv3x3_dgrad_bf16", L.ptr(dz), L.ptr(w), L.ptr(act), L.ptr(e), B, H, W, L.ptr(o1), st)
+    L.call("igm_conv3x3_bwd_bf16", L.ptr(act), L.ptr(dz), L.ptr(w), L.ptr(e), B, H, W, nblocks, L.ptr(p2), accumulate,
+           L.ptr(o2), st)
+    assert torch.equal(o1, o2) and torch.equal(p1, p2)
+
+
+@pytest.mark.parametrize("rows,n3x3,cout", [((1, 1, 1), 1, 2), ((3, 8, 5), 2, 20), ((33, 32, 31), 3, 32),
+                                            ((512, 256, 100), 1, 6), ((7, 9, 4), 0, 20)])
+def test_reduction_of_all_layers(dev, rows, n3x3, cout):
+    """igm_wgrad_reduce_layers_f32 against the layers' own reductions: two
+    orders of at most 512 float32 sums, each within 512 * 2^-24 * sum |p| at
+    worst, together 6.2e-5 of it (2e-6 are asked: 23 roundings' random walk
+    with room); rows of zeros after the last change no bit."""
+    lib, st = L.load(), L.stream_ptr()
+    kinds = [0] + [9] * n3x3 + [1]
+    nr = {0: rows[0], 9: rows[1], 1: rows[2]}
+    gen = torch.Generator().manual_seed(7)
+    parts = [torch.randn(lib.igm_wgrad_workspace_floats(t, nr[t]), generator=gen).to(dev) for t in kinds]
+    shapes = []
+    for i, t in enumerate(kinds):
+        co = cout if t == 1 else 32
+        shapes += [(max(t, 1) if t else 9) * (5 if t == 0 else 32) * co, co]
+    offs = torch.tensor([0] + list(torch.tensor(shapes).cumsum(0)), dtype=torch.int64, device=dev)
+    def reduce(extra):
+        ps = [torch.cat([p, torch.zeros(lib.igm_wgrad_workspace_floats(t, extra), device=dev)])
+              for p, t in zip(parts, kinds)]
+        mid = torch.cat(ps[1:-1]) if n3x3 else None
+        g = torch.ones(int(offs[-1]), device=dev)
+        L.call("igm_wgrad_reduce_layers_f32", n3x3, cout, nr[0] + extra, nr[9] + extra, nr[1] + extra, L.ptr(ps[0]),
+               L.ptr(mid), L.ptr(ps[-1]), 1, L.ptr(offs), L.ptr(g), st)
+        return g
+    g = reduce(0)
+    assert torch.equal(g, reduce(5))
+    for i, t in enumerate(kinds):
+        k, b = [torch.empty(shapes[2 * i + j], device=dev) for j in range(2)]
+        ka, ba = torch.empty_like(k), torch.empty_like(b)
+        for src, dk, db in ((parts[i].clone(), k, b), (parts[i].abs(), ka, ba)):
+            L.call("igm_conv_wgrad_reduce_f32", t, cout if t == 1 else 32, nr[t], L.ptr(src), 0, L.ptr(dk), L.ptr(db), st)
+        o = [int(v) for v in offs[2 * i:2 * i + 3]]
+        assert ((g[o[0]:o[1]] - 1 - k).abs() <= 2e-6 * (ka + 1)).all()
+        assert ((g[o[1]:o[2]] - 1 - b).abs() <= 2e-6 * (ba + 1)).all()
