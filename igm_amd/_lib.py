@@ -65,6 +65,7 @@ _SIGS = {
                                            VP, VP, VP, VP]),
     "igm_conv_in_fwd": (C.c_int, [VP, VP, VP, VP, VP, I64, I64, I64, VP, I32, I32, I32, VP, VP, VP, VP]),
     "igm_conv3x3_fwd_bf16": (C.c_int, [VP, VP, VP, VP, I32, I32, I32, VP, VP]),
+    "igm_conv3x3_head_fwd_bf16": (C.c_int, [VP, VP, VP, VP, VP, VP, I32, I32, I32, I32, VP, VP, VP]),
     "igm_conv3x3_pair_fwd_bf16": (C.c_int, [VP, VP, VP, VP, VP, VP, I32, I32, I32, VP, VP]),
     "igm_conv3x3_dgrad_bf16": (C.c_int, [VP, VP, VP, VP, I32, I32, I32, VP, VP]),
     "igm_conv1x1_head_fwd": (C.c_int, [VP, VP, VP, VP, I32, I32, I32, I32, VP, VP]),

@@ -67,6 +67,10 @@ struct ConvArgs {
   const float* bias[2];
   const bf16* aux;
   bf16* out;
+  const bf16* head;       // output layer (HEAD): weights [32 out][32 in], bias,
+  const float* headb;     // its result (B, H, W, cout)
+  float* Y;
+  int cout;
   const int32_t* ext;
   int B, H, W;
   ConvGeom g;
@@ -124,7 +128,12 @@ __device__ __forceinline__ uint32_t px_off(const ConvTile& t, int x, bool ok) {
 // covers whole 128-B lines (interleaved by 4 n + q instead, half lines, 1500
 // x 1500 took 74 us a layer, now 60).  Tap column s of group q is then the
 // row shifted by s - 1: nine fragments a row, whose overlap is read from L1.
-template <int MODE, int ST>
+//
+// HEAD (forward): the 1x1 output layer with it, Y = head * out + headb.  A
+// lane's 8 channels are the output layer's operand as they are, so a row's Y
+// follows its activations (a.out NULL: those are not stored).  1000 x 1000, 20
+// outputs: 38 us, 34 without the activations, where the two launches take 52.
+template <int MODE, int ST, bool HEAD>
 __global__ void __launch_bounds__(256, 2)
 conv3x3_kernel(const ConvArgs a) {
   __shared__ u32x4 wl[18][64];
@@ -141,12 +150,33 @@ conv3x3_kernel(const ConvArgs a) {
     ooff[q] = px_off(t, xl + 2 * q, xl + 2 * q < a.W);
     xin[q] = xl + 2 * q < t.nx;
   }
-  const rsrc_t rout = make_rsrc(a.out, t.bytes);
+  const rsrc_t rout = make_rsrc(a.out, !HEAD || a.out ? t.bytes : 0u);
+  // HEAD: Y of pixel slot q, output channels 16 c + 4 g .. + 3, in a row
+  const uint32_t ybytes = HEAD ? (uint32_t)a.W * a.cout * 4 : 0u;
+  const bool vec = HEAD && (a.cout % 4) == 0 && (reinterpret_cast<uintptr_t>(a.Y) & 15) == 0;
+  const int b = HEAD ? (int)(t.img / ((uint32_t)a.H * t.rowbytes)) : 0;
+  auto store_y = [&](int y, int q, int c, f32x4 v) {
+    const rsrc_t ry = make_rsrc(a.Y + ((int64_t)b * a.H + y) * a.W * a.cout, ybytes);
+    const int x = xl + 2 * q, co = 16 * c + 4 * t.g;
+    const uint32_t o = ((x < a.W) & (co < a.cout)) ? (uint32_t)(x * a.cout + co) * 4 : kOOB;
+    if (vec) {
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ry, o, 0, 0);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[e]), ry, co + e < a.cout ? o + 4 * e : kOOB, 0, 0);
+    }
+  };
   const int yv = t.x0 < t.nx ? min(t.y1, t.ny) : t.y0;  // rows y0 .. yv - 1 are computed
   for (int y = max(yv, t.y0); y < t.y1; ++y) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+    for (int q = 0; q < 4; ++q) {
       store_px<kStoreCached>(u32x4{0, 0, 0, 0}, rout, ooff[q], t.img + y * t.rowbytes);
+      if constexpr (HEAD) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) store_y(y, q, c, f32x4{0.f, 0.f, 0.f, 0.f});
+      }
+    }
   }
   if (yv <= t.y0) return;
 
@@ -154,6 +184,19 @@ conv3x3_kernel(const ConvArgs a) {
   if constexpr (MODE == 0) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) bias_r[e] = a.bias[0][8 * t.g + e];
+  }
+  bf16x8 hw[2];
+  f32x4 hb[2];
+  if constexpr (HEAD) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      hw[c] = as_bf16x8(*reinterpret_cast<const u32x4*>(a.head + (c * 16 + t.n) * kC + 8 * t.g));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int co = c * 16 + 4 * t.g + e;
+        hb[c][e] = co < a.cout ? a.headb[co] : 0.f;
+      }
+    }
   }
   // fragment f: pixels xl + f - 1, f = 0 .. 8
   uint32_t voff[9];
@@ -211,7 +254,17 @@ conv3x3_kernel(const ConvArgs a) {
       u32x4 o = __builtin_bit_cast(u32x4, h);
 #pragma unroll
       for (int i = 0; i < 4; ++i) o[i] = xin[q] ? o[i] : 0u;
-      store_px<ST>(o, rout, ooff[q], so);
+      if (!HEAD || a.out) store_px<ST>(o, rout, ooff[q], so);
+      if constexpr (HEAD) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+          f32x4 v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hw[c], as_bf16x8(o), zero, 0, 0, 0);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = xin[q] ? v[e] + hb[c][e] : 0.f;
+          store_y(y, q, c, v);
+        }
+      }
     }
   };
 
@@ -401,8 +454,32 @@ int igm_conv3x3_fwd_bf16(const void* in, const void* wpacked, const float* bias,
   const dim3 grid(a.g.blocks), block(256);
   hipStream_t st = (hipStream_t)stream;
   switch (conv_store_mode(act_bytes(B, H, W), false)) {
-    case kStoreThrough: hipLaunchKernelGGL((conv3x3_kernel<0, kStoreThrough>), grid, block, 0, st, a); break;
-    default: hipLaunchKernelGGL((conv3x3_kernel<0, kStoreCached>), grid, block, 0, st, a); break;
+    case kStoreThrough: hipLaunchKernelGGL((conv3x3_kernel<0, kStoreThrough, false>), grid, block, 0, st, a); break;
+    default: hipLaunchKernelGGL((conv3x3_kernel<0, kStoreCached, false>), grid, block, 0, st, a); break;
+  }
+  IGM_CHECK_LAUNCH();
+  return 0;
+}
+
+int igm_conv3x3_head_fwd_bf16(const void* in, const void* wpacked, const float* bias,
+                              const void* head_wpacked, const float* head_bias, const int32_t* extents,
+                              int32_t B, int32_t H, int32_t W, int32_t cout, void* out, float* Y,
+                              void* stream) {
+  IGM_CHECK_ARG(in && wpacked && bias && head_wpacked && head_bias && Y, "null pointer");
+  IGM_CHECK_ARG(in != out, "in and out must differ");
+  IGM_CHECK_ARG(cout >= 1 && cout <= kC, "cout must be in [1, 32]");
+  IGM_CHECK_ARG(B >= 1 && H >= 1 && W >= 1 && B <= 65535, "bad sizes");
+  IGM_CHECK_ARG(act_bytes(B, H, W) < (int64_t)kOOB, "activations above 2 GiB (32-bit buffer offsets)");
+  ConvArgs a = conv_args(in, wpacked, bias, nullptr, extents, B, H, W, out, kStripPx);
+  a.head = (const bf16*)head_wpacked;
+  a.headb = head_bias;
+  a.Y = Y;
+  a.cout = cout;
+  const dim3 grid(a.g.blocks), block(256);
+  hipStream_t st = (hipStream_t)stream;
+  switch (conv_store_mode(act_bytes(B, H, W), false)) {
+    case kStoreThrough: hipLaunchKernelGGL((conv3x3_kernel<0, kStoreThrough, true>), grid, block, 0, st, a); break;
+    default: hipLaunchKernelGGL((conv3x3_kernel<0, kStoreCached, true>), grid, block, 0, st, a); break;
   }
   IGM_CHECK_LAUNCH();
   return 0;
@@ -439,9 +516,9 @@ int igm_conv3x3_dgrad_bf16(const void* dz, const void* wpacked_dgrad, const void
   const dim3 grid(a.g.blocks), block(256);
   hipStream_t st = (hipStream_t)stream;
   switch (conv_store_mode(act_bytes(B, H, W), true)) {
-    case kStoreThrough: hipLaunchKernelGGL((conv3x3_kernel<1, kStoreThrough>), grid, block, 0, st, a); break;
-    case kStoreStream: hipLaunchKernelGGL((conv3x3_kernel<1, kStoreStream>), grid, block, 0, st, a); break;
-    default: hipLaunchKernelGGL((conv3x3_kernel<1, kStoreCached>), grid, block, 0, st, a); break;
+    case kStoreThrough: hipLaunchKernelGGL((conv3x3_kernel<1, kStoreThrough, false>), grid, block, 0, st, a); break;
+    case kStoreStream: hipLaunchKernelGGL((conv3x3_kernel<1, kStoreStream, false>), grid, block, 0, st, a); break;
+    default: hipLaunchKernelGGL((conv3x3_kernel<1, kStoreCached, false>), grid, block, 0, st, a); break;
   }
   IGM_CHECK_LAUNCH();
   return 0;

@@ -115,11 +115,18 @@ class CNN:
         L.call("igm_conv_in_fwd", *fptrs, fb, fr, fc, ext, B, H, W, L.ptr(self.kernel(0)),
                L.ptr(self.bias(0)), L.ptr(act), st)
         acts = [act]
-        other = None
+        Y = torch.empty((B, H, W, self.cout), dtype=torch.float32, device=dev)
+        other, headed = None, False
         li = 1
         while li < self.nl:
-            out = torch.empty_like(act) if keep or other is None else other
-            if keep or li + 1 == self.nl:
+            last = li + 1 == self.nl
+            out = None if last and not keep else (torch.empty_like(act) if keep or other is None else other)
+            if last:  # with the output layer; the activations are stored for a backward pass only
+                L.call("igm_conv3x3_head_fwd_bf16", L.ptr(act), L.ptr(self.fwd[li - 1]), L.ptr(self.bias(li)),
+                       L.ptr(self.head), L.ptr(self.bias(self.nl)), ext, B, H, W, self.cout, L.ptr(out), L.ptr(Y), st)
+                headed = True
+                li += 1
+            elif keep:
                 L.call("igm_conv3x3_fwd_bf16", L.ptr(act), L.ptr(self.fwd[li - 1]), L.ptr(self.bias(li)),
                        ext, B, H, W, L.ptr(out), st)
                 li += 1
@@ -130,9 +137,9 @@ class CNN:
             if keep:
                 acts.append(out)
             act, other = out, act
-        Y = torch.empty((B, H, W, self.cout), dtype=torch.float32, device=dev)
-        L.call("igm_conv1x1_head_fwd", L.ptr(act), L.ptr(self.head), L.ptr(self.bias(self.nl)), ext,
-               B, H, W, self.cout, L.ptr(Y), st)
+        if not headed:
+            L.call("igm_conv1x1_head_fwd", L.ptr(act), L.ptr(self.head), L.ptr(self.bias(self.nl)), ext,
+                   B, H, W, self.cout, L.ptr(Y), st)
         return (Y, acts) if keep else Y
 
     # ----------------------------------------------------------- backward --

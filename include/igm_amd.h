@@ -270,6 +270,13 @@ int igm_conv3x3_pair_fwd_bf16(const void* in, const void* w1, const float* b1, c
                               const float* b2, const int32_t* extents, int32_t B, int32_t H,
                               int32_t W, void* out, void* stream);
 
+/* igm_conv3x3_fwd_bf16 and igm_conv1x1_head_fwd on its result in one launch,
+ * bit for bit.  out NULL: the 3x3 layer's activations are not stored. */
+int igm_conv3x3_head_fwd_bf16(const void* in, const void* wpacked, const float* bias,
+                              const void* head_wpacked, const float* head_bias, const int32_t* extents,
+                              int32_t B, int32_t H, int32_t W, int32_t cout, void* out, float* Y,
+                              void* stream);
+
 /* Input gradient of a 3x3 layer (the tape through Conv2D, emulate.py:252):
  * dz_below = conv(dz, flipped W) * LeakyReLU'(act_below).
  * wpacked_dgrad: [9][32 in][32 out] bf16 with the taps reversed. */

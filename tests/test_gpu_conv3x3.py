@@ -267,3 +267,23 @@ def test_reduction_of_all_layers(dev, rows, n3x3, cout):
         o = [int(v) for v in offs[2 * i:2 * i + 3]]
         assert ((g[o[0]:o[1]] - 1 - k).abs() <= 2e-6 * (ka + 1)).all()
         assert ((g[o[1]:o[2]] - 1 - b).abs() <= 2e-6 * (ba + 1)).all()
+
+
+@pytest.mark.parametrize("cout,shift", [(20, 0), (32, 0), (2, 0), (7, 0), (20, 1)])
+@pytest.mark.parametrize("B,H,W,ext", [(1, 1, 1, None), (1, 5, 65, None), (2, 13, 64, [(13, 31), (7, 64)]),
+                                       (3, 66, 130, [(65, 130), (66, 5), (1, 1)]), (1, 300, 257, None)])
+def test_last_layer_with_the_output_layer(dev, B, H, W, ext, cout, shift):
+    """igm_conv3x3_head_fwd_bf16 runs the products of the two layers' launches:
+    equal bits, with Y on and off 16 bytes, with and without the activations."""
+    x, (w, w2), (b, b2) = case(B, H, W, dev)
+    e = None if ext is None else torch.tensor(ext, dtype=torch.int32, device=dev)
+    head, hb = w2[0].contiguous(), torch.cat([b2, b2])[:cout].contiguous()
+    st, n = L.stream_ptr(), B * H * W * cout
+    Ys = [torch.full((n + 1,), float("nan"), device=dev)[shift:shift + n] for _ in range(3)]
+    a, a2 = torch.full_like(x, float("nan")), torch.full_like(x, float("nan"))
+    L.call("igm_conv3x3_fwd_bf16", L.ptr(x), L.ptr(w), L.ptr(b), L.ptr(e), B, H, W, L.ptr(a), st)
+    L.call("igm_conv1x1_head_fwd", L.ptr(a), L.ptr(head), L.ptr(hb), L.ptr(e), B, H, W, cout, L.ptr(Ys[0]), st)
+    for out, Y in ((a2, Ys[1]), (None, Ys[2])):
+        L.call("igm_conv3x3_head_fwd_bf16", L.ptr(x), L.ptr(w), L.ptr(b), L.ptr(head), L.ptr(hb), L.ptr(e), B, H, W,
+               cout, L.ptr(out), L.ptr(Y), st)
+    assert torch.equal(a, a2) and torch.equal(Ys[0], Ys[1]) and torch.equal(Ys[0], Ys[2])
