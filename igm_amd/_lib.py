@@ -79,6 +79,10 @@ _SIGS = {
     "igm_conv_in_wgrad_partials": (C.c_int, [VP, VP, VP, VP, VP, I64, I64, I64, VP, I32, I32, I32, VP,
                                              I32, VP, I32, VP]),
     "igm_conv_wgrad_reduce_f32": (C.c_int, [I32, I32, I32, VP, I32, VP, VP, VP]),
+    "igm_cnn_fwd": (C.c_int, [I32, VP, VP, VP, VP, VP, I64, I64, I64, VP, I32, I32, I32, VP, VP, VP, VP, I32, VP, I32,
+                              VP, VP]),
+    "igm_cnn_bwd": (C.c_int, [I32, VP, VP, VP, VP, VP, VP, VP, I64, I64, I64, VP, I32, I32, I32, VP, VP, VP, I32, I32,
+                              I32, I32, VP, VP, VP, I32, VP, VP, VP, VP]),
     "igm_wgrad_reduce_layers_f32": (C.c_int, [I32, I32, I32, I32, I32, VP, VP, VP, I32, VP, VP, VP]),
     "igm_conv_in_dgrad": (C.c_int, [VP, VP, VP, I32, I32, I32, VP, VP]),
     "igm_vert_flow_kinematic_f32": (C.c_int, [I32, I32, I32, VP, VP, VP, VP, VP, VP, C.c_double, VP, VP, VP,
@@ -134,9 +138,15 @@ def ptr(t):
 
 
 def stream_ptr(stream=None):
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
+    if stream is not None:
+        return stream.cuda_stream
+    if torch.cuda.is_initialized():
+        # the current device's current stream, without a Stream object for it
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    return torch.cuda.current_stream().cuda_stream
 
 
 def call(name, *args):
-    check(getattr(load(), name)(*args))
+    rc = getattr(_lib or load(), name)(*args)
+    if rc != 0:
+        check(rc)

@@ -38,6 +38,19 @@ def glorot_uniform(shape, gen):
     return (torch.rand(shape, generator=gen, dtype=torch.float64) * 2 - 1) * lim
 
 
+class Partials:
+    """Partial sums of the weight gradients: layer 1's, the 3x3 layers' and the
+    output layer's, with their rows, in one buffer (16-B aligned parts)."""
+
+    def __init__(self, rows, n3x3, device):
+        lib = L.load()
+        n = [lib.igm_wgrad_workspace_floats(t, r) for t, r in zip((0, 9, 1), rows)]
+        self.rows = rows
+        self.buf = torch.empty(n[0] + n3x3 * n[1] + n[2], dtype=torch.float32, device=device)
+        base = self.buf.data_ptr()
+        self.ptrs = (base, base + 4 * n[0], base + 4 * (n[0] + n3x3 * n[1]))
+
+
 class CNN:
     """Parameters of the emulator (flat fp32 masters + Adam slots + bf16 operands)."""
 
@@ -108,39 +121,11 @@ class CNN:
         """fields: (f0..f4 device fp32 tensors, (fb, fr, fc) strides, B, H, W).
         Returns Y (B, H, W, 2Nz) fp32 (and the activations when keep)."""
         fptrs, (fb, fr, fc), B, H, W = fields
-        dev = self.device
-        ext = L.ptr(extents)
-        st = L.stream_ptr()
-        act = torch.empty((B, H, W, NF), dtype=torch.bfloat16, device=dev)
-        L.call("igm_conv_in_fwd", *fptrs, fb, fr, fc, ext, B, H, W, L.ptr(self.kernel(0)),
-               L.ptr(self.bias(0)), L.ptr(act), st)
-        acts = [act]
-        Y = torch.empty((B, H, W, self.cout), dtype=torch.float32, device=dev)
-        other, headed = None, False
-        li = 1
-        while li < self.nl:
-            last = li + 1 == self.nl
-            out = None if last and not keep else (torch.empty_like(act) if keep or other is None else other)
-            if last:  # with the output layer; the activations are stored for a backward pass only
-                L.call("igm_conv3x3_head_fwd_bf16", L.ptr(act), L.ptr(self.fwd[li - 1]), L.ptr(self.bias(li)),
-                       L.ptr(self.head), L.ptr(self.bias(self.nl)), ext, B, H, W, self.cout, L.ptr(out), L.ptr(Y), st)
-                headed = True
-                li += 1
-            elif keep:
-                L.call("igm_conv3x3_fwd_bf16", L.ptr(act), L.ptr(self.fwd[li - 1]), L.ptr(self.bias(li)),
-                       ext, B, H, W, L.ptr(out), st)
-                li += 1
-            else:  # two layers in one launch: the one between them is not stored
-                L.call("igm_conv3x3_pair_fwd_bf16", L.ptr(act), L.ptr(self.fwd[li - 1]), L.ptr(self.bias(li)),
-                       L.ptr(self.fwd[li]), L.ptr(self.bias(li + 1)), ext, B, H, W, L.ptr(out), st)
-                li += 2
-            if keep:
-                acts.append(out)
-            act, other = out, act
-        if not headed:
-            L.call("igm_conv1x1_head_fwd", L.ptr(act), L.ptr(self.head), L.ptr(self.bias(self.nl)), ext,
-                   B, H, W, self.cout, L.ptr(Y), st)
-        return (Y, acts) if keep else Y
+        acts = torch.empty((self.nl if keep else min(self.nl, 2), B, H, W, NF), dtype=torch.bfloat16, device=self.device)
+        Y = torch.empty((B, H, W, self.cout), dtype=torch.float32, device=self.device)
+        L.call("igm_cnn_fwd", self.nl, *fptrs, fb, fr, fc, L.ptr(extents), B, H, W, L.ptr(self.w), self.offs_host.ctypes.data,
+               L.ptr(self.fwd), L.ptr(self.head), self.cout, L.ptr(acts), 1 if keep else 0, L.ptr(Y), L.stream_ptr())
+        return (Y, list(acts.unbind(0))) if keep else Y
 
     # ----------------------------------------------------------- backward --
     def backward(self, dY, acts, fields, extents=None, nblocks=512, accumulate=False, input_grad=None,
@@ -156,32 +141,20 @@ class CNN:
         sub-batches'), and ``reduce_deferred()`` sums them into self.g once:
         one reduction per layer per batch instead of one per sub-batch."""
         fptrs, (fb, fr, fc), B, H, W = fields
-        ext = L.ptr(extents)
-        st = L.stream_ptr()
         # deferred: the sub-batches add up in the partial sums; otherwise this
         # batch's are summed (into self.g, added when accumulate) at the end
-        part, nb = self._deferred_partials(nblocks) if deferred else self._partials(nblocks, (B, H, W))
-        acc = 1 if accumulate and deferred else 0
+        part = self._deferred_partials(nblocks) if deferred else self._partials(nblocks, (B, H, W))
         nl = self.nl
-        dz = torch.empty((B, H, W, NF), dtype=torch.bfloat16, device=self.device)
-        dYb = torch.empty_like(dz)
-        L.call("igm_conv1x1_head_bwd", L.ptr(dY), L.ptr(acts[nl - 1]), L.ptr(self.kernel(nl)), ext, B, H,
-               W, self.cout, L.ptr(dz), L.ptr(dYb), st)
-        L.call("igm_conv_wgrad_partials_bf16", 1, L.ptr(acts[nl - 1]), L.ptr(dYb), ext, B, H, W, nb[1],
-               L.ptr(part[nl]), acc, st)
-        below = dYb  # reuse as the ping-pong buffer
-        for li in range(nl - 1, 0, -1):  # layer index li (0-based) is a 3x3 MFMA layer
-            L.call("igm_conv3x3_bwd_bf16", L.ptr(acts[li - 1]), L.ptr(dz), L.ptr(self.dgr[li - 1]), ext, B, H, W,
-                   nb[9], L.ptr(part[li]), acc, L.ptr(below), st)
-            dz, below = below, dz
-        L.call("igm_conv_in_wgrad_partials", *fptrs, fb, fr, fc, ext, B, H, W, L.ptr(dz), nb[0], L.ptr(part[0]),
-               acc, st)
-        if not deferred:
-            self._reduce(part, nb, accumulate)
+        dz = torch.empty((2, B, H, W, NF), dtype=torch.bfloat16, device=self.device)
         if input_grad is not None:
             assert input_grad.shape == (B, H, W, 5) and input_grad.dtype == torch.float32
             assert input_grad.is_contiguous()
-            L.call("igm_conv_in_dgrad", L.ptr(dz), L.ptr(self.kernel(0)), ext, B, H, W, L.ptr(input_grad), st)
+        at = (C.c_void_p * nl)(*[a.data_ptr() for a in acts])
+        L.call("igm_cnn_bwd", nl, L.ptr(dY), C.addressof(at), *fptrs, fb, fr, fc, L.ptr(extents), B, H, W, L.ptr(self.w),
+               self.offs_host.ctypes.data, L.ptr(self.dgr), self.cout, *part.rows, *part.ptrs, 1 if accumulate and deferred else 0,
+               dz.data_ptr(), dz.data_ptr() + dz.stride(0) * 2, L.ptr(input_grad), L.stream_ptr())
+        if not deferred:
+            self._reduce(part, accumulate)
         return self.g
 
     # The 3x3 layers' backward kernel runs one wave per SIMD, 256 blocks at
@@ -189,22 +162,18 @@ class CNN:
     WGRAD_BLOCKS = 256
 
     def _partials(self, nblocks, size=None):
-        """Partial-sum buffers of every layer (layer 0: layer 1's layout;
-        1..nl-1: 3x3, one after the other; nl: the 1x1 head) and their rows by
-        kind (0, 9 taps, 1 tap).  ``size`` (B, H, W): no more rows than there
-        are blocks with work, four pieces of 4 rows x 32 columns each (the head:
-        one of 4 x 64); at 256 x 319 the reduction takes 27 us without."""
-        lib = L.load()
-        nb = {0: nblocks, 9: min(nblocks, self.WGRAD_BLOCKS), 1: nblocks}
+        """Partial-sum buffers of every layer (layer 1; the 3x3 layers, one
+        after the other; the 1x1 head) and their rows.  ``size`` (B, H, W): no
+        more rows than there are blocks with work, four pieces of 4 rows x 32
+        columns each (the head: one of 4 x 64); at 256 x 319 the reduction
+        takes 27 us without."""
+        n_in, n_head, n_3x3 = nblocks, nblocks, min(nblocks, self.WGRAD_BLOCKS)
         if size is not None:
             B, H, W = size
             quads = B * ((H + 3) // 4)
-            work = {0: (quads * ((W + 31) // 32) + 3) // 4, 1: quads * ((W + 63) // 64)}
-            nb = {t: min(nb[t], work[1 if t == 1 else 0]) for t in nb}
-        n = {t: lib.igm_wgrad_workspace_floats(t, nb[t]) for t in nb}
-        # (each part a multiple of 16 B)
-        flat = torch.empty(n[0] + (self.nl - 1) * n[9] + n[1], dtype=torch.float32, device=self.device)
-        return flat.split([n[0]] + [n[9]] * (self.nl - 1) + [n[1]]), nb
+            work = (quads * ((W + 31) // 32) + 3) // 4
+            n_in, n_3x3, n_head = min(n_in, work), min(n_3x3, work), min(n_head, quads * ((W + 63) // 64))
+        return Partials((n_in, n_3x3, n_head), self.nl - 1, self.device)
 
     def _deferred_partials(self, nblocks):
         """The buffers of the deferred backward, kept between sub-batches."""
@@ -213,16 +182,14 @@ class CNN:
             self._part_nblocks = nblocks
         return self._part
 
-    def _reduce(self, part, nb, accumulate):
-        n3 = self.nl - 1
-        L.call("igm_wgrad_reduce_layers_f32", n3, self.cout, nb[0], nb[9], nb[1], L.ptr(part[0]),
-               L.ptr(part[1]) if n3 else None, L.ptr(part[self.nl]), 1 if accumulate else 0, L.ptr(self.offs),
-               L.ptr(self.g), L.stream_ptr())
+    def _reduce(self, part, accumulate):
+        L.call("igm_wgrad_reduce_layers_f32", self.nl - 1, self.cout, *part.rows, *part.ptrs, 1 if accumulate else 0,
+               L.ptr(self.offs), L.ptr(self.g), L.stream_ptr())
 
     def reduce_deferred(self, accumulate=False):
         """Sum the deferred partials of every layer into self.g (added to it
         when ``accumulate``) in a fixed order, in one launch."""
-        self._reduce(*self._part, accumulate)
+        self._reduce(self._part, accumulate)
         return self.g
 
     # ---------------------------------------------------------- optimizer --

@@ -24,6 +24,9 @@ def device():
 
 def as_device(x, dtype=torch.float32):
     """numpy / torch (any device) -> contiguous device tensor of ``dtype``."""
+    if (isinstance(x, torch.Tensor) and x.is_cuda and x.dtype == dtype and x.is_contiguous()
+            and x.get_device() == torch.cuda.current_device()):
+        return x
     dev = device()
     if isinstance(x, torch.Tensor):
         return x.to(device=dev, dtype=dtype).contiguous()
@@ -42,10 +45,12 @@ def velocity_outputs(U, V, thk, vert_weight, nz, write_uv=True):
     out = {n: torch.empty((Ny, Nx), dtype=dt, device=thk.device) for n in OUT_NAMES}
     Uo = torch.empty((nz, Ny, Nx), dtype=dt, device=thk.device) if write_uv else None
     Vo = torch.empty((nz, Ny, Nx), dtype=dt, device=thk.device) if write_uv else None
-    vw = (C.c_double * nz)(*[float(w) for w in np.asarray(vert_weight).ravel()[:nz]])
+    vw = np.zeros(nz)
+    w = np.asarray(vert_weight).ravel()[:nz]
+    vw[:w.size] = w
     sfx = "f32" if dt == torch.float32 else "f64"
     L.call(f"igm_velocity_outputs_{sfx}", nz, Ny, Nx, up, vp, ks, rs, cs, L.ptr(thk),
-           C.addressof(vw), L.ptr(Uo), L.ptr(Vo), *[L.ptr(out[n]) for n in OUT_NAMES],
+           vw.ctypes.data, L.ptr(Uo), L.ptr(Vo), *[L.ptr(out[n]) for n in OUT_NAMES],
            L.stream_ptr())
     out["U"], out["V"] = Uo, Vo
     return out

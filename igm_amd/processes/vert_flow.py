@@ -6,6 +6,7 @@ Supported: the default, Lagrange basis with version 2 / method "kinematic"
 (vert_flow_v2.py:17-37).  The other variants (version 1, "incompressibility",
 Legendre, SIA) raise NotImplementedError."""
 import ctypes as C
+import functools
 
 import numpy as np
 import torch
@@ -32,6 +33,13 @@ def _check(cfg):
                                   "is supported")
 
 
+@functools.lru_cache(maxsize=16)
+def _vertical_grid(nz, vs):
+    """Levels and vertical weights as arrays of doubles."""
+    return tuple((C.c_double * nz)(*[float(x) for x in np.asarray(f(nz, vs)).ravel()])
+                 for f in (compute_levels, define_vertical_weight))
+
+
 def update(cfg, state):
     """vert_flow.py:21-56."""
     _check(cfg)
@@ -40,8 +48,7 @@ def update(cfg, state):
     U, V = state.U.contiguous(), state.V.contiguous()
     assert U.dtype == torch.float32 and U.shape[0] == nz
     ny, nx = U.shape[1:]
-    levels = (C.c_double * nz)(*[float(x) for x in np.asarray(compute_levels(nz, vs)).ravel()])
-    vw = (C.c_double * nz)(*[float(x) for x in np.asarray(define_vertical_weight(nz, vs)).ravel()])
+    levels, vw = _vertical_grid(nz, vs)
     W = torch.empty_like(U)
     wb = torch.empty((ny, nx), dtype=torch.float32, device=U.device)
     ws = torch.empty_like(wb)

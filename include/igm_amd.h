@@ -345,6 +345,31 @@ int igm_conv_in_wgrad_partials(const float* f0, const float* f1, const float* f2
 int igm_conv_wgrad_reduce_f32(int32_t taps, int32_t cout, int32_t nblocks, float* partials,
                               int32_t accumulate, float* dW_hwio, float* db, void* stream);
 
+/* The forward pass of a network of nl hidden layers (layer 1, nl - 1 3x3
+ * layers) and the output layer: the launches above, in order.  w: the flat
+ * float32 parameters, layer l's kernel at w + offs[2 l], its bias at w +
+ * offs[2 l + 1] (offs: host); fwd: the 3x3 layers' packed kernels one after
+ * the other; acts: nl activations (B, H, W, 32) bf16 one after the other, all
+ * stored when keep, else two that take turns (one for nl <= 2). */
+int igm_cnn_fwd(int32_t nl, const float* f0, const float* f1, const float* f2, const float* f3,
+                const float* f4, int64_t fb, int64_t fr, int64_t fc, const int32_t* extents,
+                int32_t B, int32_t H, int32_t W, const float* w, const int64_t* offs,
+                const void* fwd, const void* head, int32_t cout, void* acts, int32_t keep, float* Y,
+                void* stream);
+
+/* Its backward pass from dY: the partial sums of every layer's weight gradient
+ * (written, or added to when accumulate; see igm_wgrad_reduce_layers_f32) and,
+ * if input_grad, the gradient of the 5 fields.  acts: nl host pointers; dgr:
+ * the 3x3 layers' packed data gradient kernels; dz0, dz1: two scratch
+ * activations. */
+int igm_cnn_bwd(int32_t nl, const float* dY, const void* const* acts, const float* f0,
+                const float* f1, const float* f2, const float* f3, const float* f4, int64_t fb,
+                int64_t fr, int64_t fc, const int32_t* extents, int32_t B, int32_t H, int32_t W,
+                const float* w, const int64_t* offs, const void* dgr, int32_t cout,
+                int32_t nblocks_in, int32_t nblocks_3x3, int32_t nblocks_head, float* part_in,
+                float* part_3x3, float* part_head, int32_t accumulate, void* dz0, void* dz1,
+                float* input_grad, void* stream);
+
 /* The reduction of every layer of a network in one launch: the partial sums
  * of layer 1 (nblocks_in rows), of the nlayers3x3 3x3 layers (nblocks_3x3 rows
  * each, one layer's workspace after the other) and of the output layer

@@ -287,3 +287,49 @@ def test_last_layer_with_the_output_layer(dev, B, H, W, ext, cout, shift):
         L.call("igm_conv3x3_head_fwd_bf16", L.ptr(x), L.ptr(w), L.ptr(b), L.ptr(head), L.ptr(hb), L.ptr(e), B, H, W,
                cout, L.ptr(out), L.ptr(Y), st)
     assert torch.equal(a, a2) and torch.equal(Ys[0], Ys[1]) and torch.equal(Ys[0], Ys[2])
+
+
+@pytest.mark.parametrize("nl", [1, 2, 3, 4])
+def test_network_passes_equal_their_launches(dev, nl):
+    """igm_cnn_fwd and igm_cnn_bwd make the launches of every layer in order:
+    the bits of the calls made one by one, for odd and even numbers of layers."""
+    from igm_amd import emulator as EM
+    B, H, W, nz = 2, 21, 70, 3
+    gen = torch.Generator().manual_seed(nl)
+    X = torch.rand((B, H, W, 5), generator=gen).to(dev)
+    ext = torch.tensor([[21, 70], [9, 33]], dtype=torch.int32, device=dev)
+    cnn, fields, st = EM.CNN(nz, nl, seed=3), EM.nhwc_fields(X), L.stream_ptr()
+    fp, (fb, fr, fc) = fields[0], fields[1]
+    Y, acts = cnn.forward(fields, extents=ext, keep=True)
+    ref = [torch.empty((B, H, W, 32), dtype=torch.bfloat16, device=dev) for _ in range(nl)]
+    L.call("igm_conv_in_fwd", *fp, fb, fr, fc, L.ptr(ext), B, H, W, L.ptr(cnn.kernel(0)), L.ptr(cnn.bias(0)),
+           L.ptr(ref[0]), st)
+    for i in range(1, nl):
+        L.call("igm_conv3x3_fwd_bf16", L.ptr(ref[i - 1]), L.ptr(cnn.fwd[i - 1]), L.ptr(cnn.bias(i)), L.ptr(ext), B, H,
+               W, L.ptr(ref[i]), st)
+    Yr = torch.empty_like(Y)
+    L.call("igm_conv1x1_head_fwd", L.ptr(ref[-1]), L.ptr(cnn.head), L.ptr(cnn.bias(nl)), L.ptr(ext), B, H, W, 2 * nz,
+           L.ptr(Yr), st)
+    assert torch.equal(Y, Yr) and torch.equal(cnn.forward(fields, extents=ext), Yr)
+    assert all(torch.equal(a, r) for a, r in zip(acts, ref))
+
+    dY, gX, g = torch.randn(Y.shape, generator=gen).to(dev), torch.empty_like(X), torch.empty_like(X)
+    got = cnn.backward(dY, acts, fields, extents=ext, input_grad=gX, nblocks=8).clone()
+    dz, below = torch.empty_like(ref[0]), torch.empty_like(ref[0])
+    kinds = [0] + [9] * (nl - 1) + [1]
+    parts = [torch.empty(L.load().igm_wgrad_workspace_floats(t, 8), device=dev) for t in kinds]
+    L.call("igm_conv1x1_head_bwd", L.ptr(dY), L.ptr(ref[-1]), L.ptr(cnn.kernel(nl)), L.ptr(ext), B, H, W, 2 * nz,
+           L.ptr(dz), L.ptr(below), st)
+    L.call("igm_conv_wgrad_partials_bf16", 1, L.ptr(ref[-1]), L.ptr(below), L.ptr(ext), B, H, W, 8, L.ptr(parts[nl]), 0,
+           st)
+    for i in range(nl - 1, 0, -1):
+        L.call("igm_conv3x3_bwd_bf16", L.ptr(ref[i - 1]), L.ptr(dz), L.ptr(cnn.dgr[i - 1]), L.ptr(ext), B, H, W, 8,
+               L.ptr(parts[i]), 0, L.ptr(below), st)
+        dz, below = below, dz
+    L.call("igm_conv_in_wgrad_partials", *fp, fb, fr, fc, L.ptr(ext), B, H, W, L.ptr(dz), 8, L.ptr(parts[0]), 0, st)
+    L.call("igm_conv_in_dgrad", L.ptr(dz), L.ptr(cnn.kernel(0)), L.ptr(ext), B, H, W, L.ptr(g), st)
+    mid = torch.cat(parts[1:nl]) if nl > 1 else None
+    out = torch.empty_like(cnn.g)
+    L.call("igm_wgrad_reduce_layers_f32", nl - 1, 2 * nz, 8, 8, 8, L.ptr(parts[0]), L.ptr(mid), L.ptr(parts[nl]), 0,
+           L.ptr(cnn.offs), L.ptr(out), st)
+    assert torch.equal(got, out) and torch.equal(gX, g)
