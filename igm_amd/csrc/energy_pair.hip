@@ -43,57 +43,6 @@ constexpr int kOneIter = 0;   // one iteration
 constexpr int kStageA = 1;    // two iterations, stage A only
 constexpr int kPairStep = 2;  // two iterations, stages A and B
 
-// Prologue of a device-driven solve pass (a.alpha_tab set), done by every
-// block.  The state *es_in is the one the previous pass started from, so the
-// previous pass's iteration count is recomputed from it exactly as that pass
-// decided it; those iterations are then accounted in order (their COSTs from
-// the previous partials, the EarlyStopping rule of iceflow/utils.py:92-111
-// on a private copy).  Block 0 writes the new state to *es_out and the COSTs
-// to cost_hist.  Returns the iterations this pass runs (0, 1 or 2) and its
-// first iteration in *it0.
-__device__ int solve_prologue(const PassArgs<float>& a, bool block0, int* it0) {
-  IgmEarlyStop st = *a.es_in;
-  const int f_prev = st.iters_done;
-  const int c_prev = a.prev_partials != nullptr ? pass_iterations(st, f_prev, a.nbitmax) : 0;
-  // The previous pass's COSTs can raise `wait` by at most one each (the
-  // first only sets the best when there is none).  If even then wait + 1
-  // stays below patience, the rule stops nowhere in that pass and cannot stop
-  // at this pass's first iteration: the count below is pass_iterations' for
-  // any COSTs.  Only block 0, which writes the state and the COST history,
-  // then needs the sums; every other block starts its work at once.
-  const int max_wait = st.wait + (st.has_best ? c_prev : (c_prev > 0 ? c_prev - 1 : 0));
-  if (!block0 && !st.stopped && max_wait + 1 < st.patience) {
-    const int f = f_prev + c_prev;
-    *it0 = f;
-    if (a.finalize_only || f >= a.nbitmax) return 0;
-    return f + 1 < a.nbitmax ? 2 : 1;
-  }
-  for (int t = 0; t < c_prev; ++t) {
-    double r[3];
-    block_sum_partials(a.prev_partials + 3 * t, a.prev_nblk, 6, r);
-    const double cost = (r[0] + r[1]) + r[2];
-    es_apply(st, cost, f_prev + t);
-    if (block0 && threadIdx.x == 0) {
-      a.fin_out[0] = r[0];
-      a.fin_out[1] = r[1];
-      a.fin_out[2] = r[2];
-      a.fin_out[3] = cost;
-      if (a.cost_hist != nullptr) a.cost_hist[f_prev + t] = cost;
-    }
-  }
-  if (c_prev > 0) st.passes += 1;
-  if (block0 && threadIdx.x == 0) *a.es_out = st;
-  *it0 = st.iters_done;
-  return a.finalize_only ? 0 : pass_iterations(st, st.iters_done, a.nbitmax);
-}
-
-// Velocity layouts of a pass's input and output (template bits): planar, U
-// and V in two (Nz, Ny, Nx) buffers, or interleaved, one (Nz, Ny, Nx, 2)
-// buffer holding (U, V) per node and level -- one 8-B access where planar
-// takes two 4-B ones.  A solve keeps its intermediate fields interleaved.
-constexpr int kInInterleaved = 1;
-constexpr int kOutInterleaved = 2;
-
 template <int NZ, int LAYOUT>
 __global__ void __launch_bounds__(kPassBlock)
 energy_pair_kernel(const PassArgs<float> a) {
@@ -447,6 +396,7 @@ int pair_impl(int nz, int Ny, int Nx, const float* U, const float* V, const floa
   a.omb2 = 1.0f - float(adam1->beta2);
   a.eps = float(adam1->epsilon);
   hipStream_t st = (hipStream_t)stream;
+  if (g.team) return team_launch(nz, layout, g.blocks, a, st);
   switch (nz) {
 #define IGM_PAIR_CASE(N)                                                                                \
   case N:                                                                                               \

@@ -254,6 +254,16 @@ struct CellEnergy {
 // inputs depend on each other's outputs (the two-iteration pass).
 //
 // THIRD (float64): both powers are within 1e-12 of -1/3 (pow_third).
+//
+// With SplitRow in the carry's place a sweep does without the carry of cell
+// row jc - 1: X and Z of scatter are kept, for (carry - Z) + X later, and the
+// carry for the next row is X + Z.
+template <typename T, int NZ>
+struct SplitRow {
+  T x[NZ], z[NZ];
+  __device__ __forceinline__ T carry(int k) const { return x[k] + z[k]; }
+  __device__ __forceinline__ T gradient(int k, T carry) const { return (carry - z[k]) + x[k]; }
+};
 template <typename T, int NZ, bool THIRD = false>
 struct LevelSweep {
   const PassArgs<T>& a;
@@ -282,6 +292,16 @@ struct LevelSweep {
     return g;
   }
 
+  __device__ __forceinline__ static void split(SplitRow<T, NZ>& r, int k, T gx_, T gy_, T gs_) {
+    const T A = gs_ - gx_, B = gs_ + gx_;
+    r.x[k] = A + lane_from_left(B);
+    r.z[k] = gy_ + lane_from_left(gy_);
+  }
+  template <typename Emit>
+  __device__ __forceinline__ void out(int k, SplitRow<T, NZ>& cu, SplitRow<T, NZ>& cv, Emit&&) {
+    split(cu, k, g_ux, g_uy, g_su);
+    split(cv, k, g_vx, g_vy, g_sv);
+  }
   template <typename Emit>
   __device__ __forceinline__ void out(int k, T (&cu)[NZ], T (&cv)[NZ], Emit&& emit) {
     const T g_u = scatter(cu[k], g_ux, g_uy, g_su);
@@ -293,9 +313,9 @@ struct LevelSweep {
   // Multiply-adds are fused within one expression only, never across
   // statements: the fusion then follows the source, not the surrounding
   // kernel, and every kernel that runs this sweep rounds the same way.
-  template <typename Emit>
-  __device__ __forceinline__ void level(int k, T upk, T vpk, T uck, T vck, T (&cu)[NZ],
-                                        T (&cv)[NZ], Emit&& emit) {
+  template <typename Carry, typename Emit>
+  __device__ __forceinline__ void level(int k, T upk, T vpk, T uck, T vck, Carry& cu, Carry& cv,
+                                        Emit&& emit) {
 #pragma clang fp contract(on)
     const T su = upk + uck, du = uck - upk;
     const T sv = vpk + vck, dv = vck - vpk;
@@ -370,8 +390,8 @@ struct LevelSweep {
   }
 
   // Emits level NZ-1 and returns the cell's (shear, sliding, gravity) energy.
-  template <typename Emit>
-  __device__ __forceinline__ CellEnergy<T> finish(T (&cu)[NZ], T (&cv)[NZ], Emit&& emit) {
+  template <typename Carry, typename Emit>
+  __device__ __forceinline__ CellEnergy<T> finish(Carry& cu, Carry& cv, Emit&& emit) {
 #pragma clang fp contract(on)
     out(NZ - 1, cu, cv, emit);
     return {w * c_sh, c_sl, gx * wsu + gy * wsv};
@@ -456,6 +476,7 @@ inline int pair_target_waves() {
 
 struct PassGeom {
   int nstrips, nrowblk, blocks;
+  bool team = false;  // two iterations by teams of four waves (energy_team.hip)
 };
 // Strips of `strip_out` owned columns, their rows split evenly into nrowblk
 // blocks.  `full`: waves that run at once; `extra`: steps of a wave beyond its
@@ -493,9 +514,81 @@ inline PassGeom one_pass_geom(int nbatch, int Ny, int Nx) {
   if (env || Ny >= kFullRows * g.nrowblk) return g;
   return pass_geom(nbatch, Ny, Nx, kStripOut, kTargetWaves / 2, 1, env);
 }
+//
+// The two-iteration pass goes to teams of four waves (energy_team.hip) where
+// they are done in kTeamSteps steps, of 4 s - 3 rows in s steps, in one round of
+// blocks: a launch of 100 x 100 (one step) takes 10.9 us, 19.1 as a march, 200 x
+// 251 (two) 18.9 and 21.9, 300 x 300 (three) 26.5 and 27.7; 400 x 400 (four)
+// 36.4 and 33.8.
+constexpr int kTeamSteps = 3;
 inline PassGeom pair_pass_geom(int Ny, int Nx) {
-  return pass_geom(1, Ny, Nx, kPairOut, kPairTargetWaves, 2, pair_target_waves());
+  const int env = pair_target_waves();
+  const PassGeom g = pass_geom(1, Ny, Nx, kPairOut, kPairTargetWaves, 2, env);
+  const int room = kPairTargetWaves / kWavesPerBlock / g.nstrips;  // row blocks that run at once
+  if (env || room < 1) return g;
+  PassGeom t{g.nstrips, room < Ny ? room : Ny, 0, true};
+  const int steps = ((Ny + t.nrowblk - 1) / t.nrowblk + 3 + 3) / 4;
+  // fewer blocks where the steps stay as many
+  t.nrowblk = (Ny + 4 * steps - 4) / (4 * steps - 3);
+  t.blocks = t.nstrips * t.nrowblk;
+  return steps <= kTeamSteps ? t : g;
 }
+
+// ------------------------------------------- two iterations per launch --
+//
+// Prologue of a device-driven solve pass (a.alpha_tab set), done by every
+// block.  The state *es_in is the one the previous pass started from, so the
+// previous pass's iteration count is recomputed from it exactly as that pass
+// decided it; those iterations are then accounted in order (their COSTs from
+// the previous partials, the EarlyStopping rule of iceflow/utils.py:92-111
+// on a private copy).  Block 0 writes the new state to *es_out and the COSTs
+// to cost_hist.  Returns the iterations this pass runs (0, 1 or 2) and its
+// first iteration in *it0.
+__device__ inline int solve_prologue(const PassArgs<float>& a, bool block0, int* it0) {
+  IgmEarlyStop st = *a.es_in;
+  const int f_prev = st.iters_done;
+  const int c_prev = a.prev_partials != nullptr ? pass_iterations(st, f_prev, a.nbitmax) : 0;
+  // The previous pass's COSTs can raise `wait` by at most one each (the
+  // first only sets the best when there is none).  If even then wait + 1
+  // stays below patience, the rule stops nowhere in that pass and cannot stop
+  // at this pass's first iteration: the count below is pass_iterations' for
+  // any COSTs.  Only block 0, which writes the state and the COST history,
+  // then needs the sums; every other block starts its work at once.
+  const int max_wait = st.wait + (st.has_best ? c_prev : (c_prev > 0 ? c_prev - 1 : 0));
+  if (!block0 && !st.stopped && max_wait + 1 < st.patience) {
+    const int f = f_prev + c_prev;
+    *it0 = f;
+    if (a.finalize_only || f >= a.nbitmax) return 0;
+    return f + 1 < a.nbitmax ? 2 : 1;
+  }
+  for (int t = 0; t < c_prev; ++t) {
+    double r[3];
+    block_sum_partials(a.prev_partials + 3 * t, a.prev_nblk, 6, r);
+    const double cost = (r[0] + r[1]) + r[2];
+    es_apply(st, cost, f_prev + t);
+    if (block0 && threadIdx.x == 0) {
+      a.fin_out[0] = r[0];
+      a.fin_out[1] = r[1];
+      a.fin_out[2] = r[2];
+      a.fin_out[3] = cost;
+      if (a.cost_hist != nullptr) a.cost_hist[f_prev + t] = cost;
+    }
+  }
+  if (c_prev > 0) st.passes += 1;
+  if (block0 && threadIdx.x == 0) *a.es_out = st;
+  *it0 = st.iters_done;
+  return a.finalize_only ? 0 : pass_iterations(st, st.iters_done, a.nbitmax);
+}
+
+// Velocity layouts of a pass's input and output (template bits): planar, U
+// and V in two (Nz, Ny, Nx) buffers, or interleaved, one (Nz, Ny, Nx, 2)
+// buffer holding (U, V) per node and level -- one 8-B access where planar
+// takes two 4-B ones.  A solve keeps its intermediate fields interleaved.
+constexpr int kInInterleaved = 1;
+constexpr int kOutInterleaved = 2;
+
+// The two-iteration pass by teams of waves (energy_team.hip).
+int team_launch(int nz, int layout, int blocks, const PassArgs<float>& a, hipStream_t st);
 
 // Fills the physics and vertical-grid fields of the argument block (host).
 template <typename T>
