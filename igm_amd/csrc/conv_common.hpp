@@ -32,6 +32,120 @@ __device__ __forceinline__ const u32x4* conv_weight_frag(const bf16* wt, int n, 
   return reinterpret_cast<const u32x4*>(wt + ((tap * kC + 8 * (n >> 2) + 4 * cb + (n & 3)) * kC + 8 * g));
 }
 
+// A layer's rows, split over the n waves of one launch by its kernel itself:
+// the strips of kPx columns one after the other, their rows in groups of kRows,
+// and every wave an equal range of that sequence, none a group longer than
+// another's.  Of a batch of uneven entries only what is inside the extents
+// counts, which the host does not know.  A range that runs on into the next
+// strip costs another start of the march; without extents every strip is cut
+// into `chunks` ranges of its own where that is no worse (strip_chunks).
+struct StripRange {
+  int b, x0;   // batch entry, first column
+  int y0, y1;  // rows
+  int ny, nx;  // the entry's extent
+};
+template <int kPx, int kRows>
+struct StripShare {
+  const int32_t* ext;
+  int B, H, W;
+  int u, hi;    // units (groups of rows) left to this wave
+  int b, base;  // entry of unit u and that entry's first unit
+
+  // sum over this and the lower lanes
+  __device__ __forceinline__ static int scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // row_shr 1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast 15, 31
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
+    return v;
+  }
+  __device__ __forceinline__ void units(int e, int& q, int& strips, int& ny, int& nx) const {
+    extent_of(ext, e, H, W, ny, nx);
+    q = (max(ny, 0) + kRows - 1) / kRows;
+    strips = (max(nx, 0) + kPx - 1) / kPx;
+  }
+  __device__ __forceinline__ void range(int total, int w, int n) {
+    const int k = total / n, r = total % n;
+    u = w * k + min(w, r);
+    hi = u + k + (w < r ? 1 : 0);
+  }
+  // wave w of n
+  __device__ __forceinline__ StripShare(const int32_t* ext_, int B_, int H_, int W_, int chunks, int w, int n)
+      : ext(ext_), B(B_), H(H_), W(W_), u(0), hi(0), b(0), base(0) {
+    int q, strips, ny, nx;
+    if (ext == nullptr) {
+      units(0, q, strips, ny, nx);
+      if (chunks > 0) {
+        const int strip = w / chunks, k = w % chunks;
+        if (strip >= B * strips) return;
+        u = strip * q + k * (q / chunks) + min(k, q % chunks);
+        hi = u + q / chunks + (k < q % chunks ? 1 : 0);
+      } else {
+        range(B * strips * q, w, n);
+      }
+      b = u / (strips * q);
+      base = b * strips * q;
+      return;
+    }
+    // 64 entries at a time, one per lane: their units and the sum up to them
+    int v = 0, p = 0;
+    auto entries = [&](int e0) {
+      const int e = e0 + (threadIdx.x & 63);
+      v = 0;
+      if (e < B) {
+        units(e, q, strips, ny, nx);
+        v = q * strips;
+      }
+      p = scan(v);
+      return __builtin_amdgcn_readlane(p, 63);
+    };
+    int total = 0;
+    for (int e0 = 0; e0 < B; e0 += 64) total += entries(e0);
+    range(total, w, n);
+    if (u >= hi) return;
+    int e0 = 0;
+    if (B > 64) {
+      for (int t; base + (t = entries(e0)) <= u; e0 += 64) base += t;
+    }
+    const int f = __builtin_ctzll(__ballot(base + p > u));
+    b = e0 + f;
+    base += __builtin_amdgcn_readlane(p, f) - __builtin_amdgcn_readlane(v, f);
+  }
+  // (a loop over the ranges leaves out empty ones, which there are none of:
+  // without that test the compiler spills the accumulators around next)
+  __device__ __forceinline__ bool more() const { return u < hi; }
+  __device__ __forceinline__ StripRange next() {
+    StripRange s;
+    int q, strips;
+    units(b, q, strips, s.ny, s.nx);
+    while (u - base >= q * strips) {  // the next entry with rows
+      base += q * strips;
+      units(++b, q, strips, s.ny, s.nx);
+    }
+    const int i = (u - base) / q, g = (u - base) % q, k = min(q - g, hi - u);
+    s.b = b;
+    s.x0 = i * kPx;
+    s.y0 = g * kRows;
+    s.y1 = min((g + k) * kRows, s.ny);
+    u += k;
+    return s;
+  }
+};
+
+// The ranges a strip of a batch without extents is cut into, for n waves, or
+// 0 for one sequence of all strips: whichever leaves the longest wave the
+// fewest rows, with `start` rows' time for each start of the march.
+inline int strip_chunks(const int32_t* ext, int B, int H, int W, int px, int rows, int start, int n) {
+  if (ext != nullptr) return 0;
+  const int64_t strips = (int64_t)B * ((W + px - 1) / px), q = ((int64_t)H + rows - 1) / rows;
+  const int64_t chunks = n / strips < q ? n / strips : q;
+  if (chunks < 1) return 0;
+  const int64_t apart = (q + chunks - 1) / chunks * rows + start, joined = (strips * q + n - 1) / n * rows + 2 * start;
+  return apart <= joined ? (int)chunks : 0;
+}
+
 // cache policy of a kernel's stores: cached, non-temporal, written through
 constexpr int kStoreCached = 0, kStoreStream = 2, kStoreThrough = 16;
 

@@ -24,6 +24,7 @@
 namespace igm {
 
 constexpr int kWgPx = 32;                 // columns of a wave's strip: the K of one product
+constexpr int kWgRows = 4;                // rows of a round of the march
 constexpr int kWgEntries = 9 * kC * kC + kC;  // floats of a block's partial sums
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -44,7 +45,7 @@ __device__ __forceinline__ bf16x8 transposed(const bf16* s, int p, int cb) {
 // The sums of a block's four waves, in order, in the lanes' own layout: entry
 // ((tap * 4 + block) * 64 + lane) * 4 + e, then the bias.
 __device__ __forceinline__ void wave_sums(const f32x4 (&acc)[9][2][2], const f32x4 (&accb)[2],
-                                          f32x4 (&sums)[4][kWgEntries / 4], int accumulate, float* partials) {
+                                          f32x4 (&sums)[4][kWgEntries / 4], int blk, int accumulate, float* partials) {
   const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4, wave = threadIdx.x >> 6;
   __syncthreads();
 #pragma unroll
@@ -56,7 +57,7 @@ __device__ __forceinline__ void wave_sums(const f32x4 (&acc)[9][2][2], const f32
     for (int c = 0; c < 2; ++c) sums[wave][9 * kC * kC / 4 + 4 * c + g] = accb[c];
   }
   __syncthreads();
-  f32x4* P = reinterpret_cast<f32x4*>(partials + (int64_t)blockIdx.x * kWgEntries);
+  f32x4* P = reinterpret_cast<f32x4*>(partials + (int64_t)blk * kWgEntries);
   constexpr int kPer = (kWgEntries / 4 + 255) / 256;
   f32x4 prev[kPer];
 #pragma unroll
@@ -77,8 +78,7 @@ __device__ __forceinline__ void wave_sums(const f32x4 (&acc)[9][2][2], const f32
 
 __global__ void __launch_bounds__(256, 1)
 wgrad3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const int32_t* __restrict__ ext,
-                int B, int H, int W, int nstrips, int nchunk, int rows, int accumulate,
-                float* __restrict__ partials) {
+                int B, int H, int W, int chunks, int accumulate, float* __restrict__ partials) {
   constexpr int kRing = 4;  // rows of each operand in flight from memory
   // rows in transposition, later the waves' sums
   constexpr int kStage = (kWgPx + 16 + kWgPx) * kC;
@@ -88,6 +88,7 @@ wgrad3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const
   } sm;
   const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int blk = xcd_remap(blockIdx.x, gridDim.x), wid = blk * 4 + wave, nw = gridDim.x * 4;
   bf16* sa = sm.rows[wave];                       // activation row: pixels x0 - 1 .. x0 + 32
   bf16* sz = sa + (kWgPx + 16) * kC;       // dz row: pixels x0 .. x0 + 31
   const uint32_t bytes = (uint32_t)((int64_t)B * H * W * kC * 2);
@@ -103,15 +104,10 @@ wgrad3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const
 #pragma unroll
   for (int e = 0; e < 8; ++e) ones[e] = f2bf(1.f);
 
-  const int ntask = B * nstrips * nchunk;
-  for (int task = blockIdx.x * 4 + wave; task < ntask; task += gridDim.x * 4) {
-    const int x0 = (task % nstrips) * kWgPx;
-    const int y0 = ((task / nstrips) % nchunk) * rows;
-    const int b = task / (nstrips * nchunk);
-    int ny, nx;
-    extent_of(ext, b, H, W, ny, nx);
-    const int y1 = min(y0 + rows, ny);
-    if (x0 >= nx || y0 >= y1) continue;
+  StripShare<kWgPx, kWgRows> share(ext, B, H, W, chunks, wid, nw);
+  while (share.more()) {
+    const auto [b, x0, y0, y1, ny, nx] = share.next();
+    if (y0 >= y1) continue;
     const uint32_t img = (uint32_t)b * H * rowbytes;
     // a lane's 16 B of a row: pixel lane / 4 of 16, chunk lane % 4
     const int px = lane >> 2;
@@ -171,7 +167,7 @@ wgrad3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const
     }
   }
 
-  wave_sums(acc, accb, sm.sums, accumulate, partials);
+  wave_sums(acc, accb, sm.sums, blk, accumulate, partials);
 }
 
 // The weight gradient and the data gradient, below = conv(dz, wt) * (act > 0 ?
@@ -184,14 +180,19 @@ wgrad3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const
 // fragments serve both output rows, a tap's weights are kept for the second.
 //
 // What bounds it: at 1000 x 1000 the memory, 192 MB in 46 us, 4.2 TB/s (the two
-// kernels: 57); 8 x 496 x 496 padded patches 74 us (93), 256 x 319 11.4 us
-// (15.8), where a wave has four rows and as many steps to fill and drain.  With
-// one row per step, the weights read for every row and operands in registers
-// that spilled, 1000 x 1000 took 69 us.
+// kernels: 57); 256 x 319 11.4 us (15.8), where a wave has four rows and as many
+// steps to fill and drain.  With one row per step, the weights read for every
+// row and operands in registers that spilled, 1000 x 1000 took 69 us.
+//
+// Batches of uneven patches take as long as the wave with the most rows, about
+// 1 us a row and 8 us more.  Split by StripShare, 8 patches of 197 .. 294 cells
+// take 37 us and of 302 .. 394 cells 50 us; with equal blocks of rows of the
+// padded batch, dealt out in turn, 58 and 75.  At 410 .. 496 cells memory bounds
+// it again, and neighbouring strips out of step cost 6 us: 88, then 82.
 template <int ST>
 __global__ void __launch_bounds__(256, 1)
 bwd3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const bf16* __restrict__ wt,
-              const int32_t* __restrict__ ext, int B, int H, int W, int nstrips, int nchunk, int rows, int accumulate,
+              const int32_t* __restrict__ ext, int B, int H, int W, int chunks, int accumulate,
               bf16* __restrict__ below, float* __restrict__ partials) {
   constexpr int kRowPx = kWgPx + 16;  // an LDS row: pixels x0 - 1 .. x0 + 32 (and 14 unused)
   // four rows of each operand and the weights, later the waves' sums
@@ -204,6 +205,7 @@ bwd3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const b
   } sm;
   const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int blk = xcd_remap(blockIdx.x, gridDim.x), wid = blk * 4 + wave, nw = gridDim.x * 4;
   const uint32_t bytes = (uint32_t)((int64_t)B * H * W * kC * 2);
   const uint32_t rowbytes = (uint32_t)W * kC * 2;
   for (int f = threadIdx.x >> 6; f < 18; f += 4) sm.in.w[f][lane] = *conv_weight_frag(wt, n, g, f >> 1, f & 1);
@@ -219,14 +221,21 @@ bwd3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const b
 #pragma unroll
   for (int e = 0; e < 8; ++e) ones[e] = f2bf(1.f);
 
-  const int ntask = B * nstrips * nchunk;
-  for (int task = blockIdx.x * 4 + wave; task < ntask; task += gridDim.x * 4) {
-    const int x0 = (task % nstrips) * kWgPx;
-    const int y0 = ((task / nstrips) % nchunk) * rows;
-    const int b = task / (nstrips * nchunk);
-    int ny, nx;
-    extent_of(ext, b, H, W, ny, nx);
-    const int y1 = x0 < nx ? min(y0 + rows, ny) : y0;
+  if (ext != nullptr) {  // zeros outside the extents' strips, a row at a time
+    const rsrc_t ro = make_rsrc(below, bytes);
+    for (int r = wid; r < B * H; r += nw) {
+      int ny, nx;
+      extent_of(ext, r / H, H, W, ny, nx);
+      const int x0 = r % H < ny ? (max(nx, 0) + kWgPx - 1) / kWgPx * kWgPx : 0;
+      for (int x = x0 + (lane >> 2); x < W; x += 16)
+        __builtin_amdgcn_raw_buffer_store_b128(u32x4{0, 0, 0, 0}, ro,
+                                               (uint32_t)r * rowbytes + (uint32_t)(x * kC * 2 + (lane & 3) * 16), 0, 0);
+    }
+  }
+  StripShare<kWgPx, kWgRows> share(ext, B, H, W, chunks, wid, nw);
+  while (share.more()) {
+    const auto [b, x0, y0, y1, ny, nx] = share.next();
+    if (y0 >= y1) continue;
     const uint32_t img = (uint32_t)b * H * rowbytes;
     uint32_t oo[2];  // data gradient: pixel x0 + 16 q + n, channels 8 g .. 8 g + 7
     bool xin[2];
@@ -236,13 +245,6 @@ bwd3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const b
       oo[q] = x < W ? (uint32_t)(x * kC + 8 * g) * 2 : kOOB;
       xin[q] = x < nx;
     }
-    for (int y = max(y1, y0); y < min(y0 + rows, H); ++y) {  // rows outside the extent
-      const rsrc_t ro = make_rsrc(below, bytes);
-#pragma unroll
-      for (int q = 0; q < 2; ++q)
-        __builtin_amdgcn_raw_buffer_store_b128(u32x4{0, 0, 0, 0}, ro, oo[q] + img + (uint32_t)y * rowbytes, 0, 0);
-    }
-    if (y0 >= y1) continue;
     // a lane's 16 B of a row: pixel lane / 4 of 16, chunk lane % 4
     const int px = lane >> 2;
     auto off = [&](int x, bool ok) { return (ok & (x >= 0) & (x < nx)) ? (uint32_t)(x * kC * 2 + (lane & 3) * 16) : kOOB; };
@@ -394,7 +396,7 @@ bwd3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const b
       step(5, j + 2);
     }
   }
-  wave_sums(acc, accb, sm.sums, accumulate, partials);
+  wave_sums(acc, accb, sm.sums, blk, accumulate, partials);
 }
 
 // Layer 1 (5 float32 fields -> 32): dW1[tap][ci][co] = sum_p X[p + delta_tap][ci] * dz1[p][co].
@@ -416,8 +418,8 @@ constexpr int kInOut = 9 * kCin * kC + kC;     // floats of a block's partial su
 __global__ void __launch_bounds__(256, 2)
 conv_in_wgrad_kernel(const float* __restrict__ f0, const float* __restrict__ f1, const float* __restrict__ f2,
                      const float* __restrict__ f3, const float* __restrict__ f4, int64_t fb, int64_t fr, int64_t fc,
-                     const bf16* __restrict__ dz, const int32_t* __restrict__ ext, int B, int H, int W, int nstrips,
-                     int nchunk, int rows, int accumulate, float* __restrict__ partials) {
+                     const bf16* __restrict__ dz, const int32_t* __restrict__ ext, int B, int H, int W, int chunks, int accumulate,
+                     float* __restrict__ partials) {
   constexpr int kRing = 4;         // rows of each operand in flight from memory
   constexpr int kXpx = kWgPx + 2;  // pixels x0 - 1 .. x0 + 32
   constexpr int kStage = (kXpx * kXc + kWgPx * kC);
@@ -427,6 +429,7 @@ conv_in_wgrad_kernel(const float* __restrict__ f0, const float* __restrict__ f1,
   } sm;
   const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int blk = xcd_remap(blockIdx.x, gridDim.x), wid = blk * 4 + wave, nw = gridDim.x * 4;
   bf16* sx = sm.rows[wave];
   bf16* sz = sx + kXpx * kXc;
   const uint32_t bytes = (uint32_t)((int64_t)B * H * W * kC * 2);
@@ -437,15 +440,10 @@ conv_in_wgrad_kernel(const float* __restrict__ f0, const float* __restrict__ f1,
 #pragma unroll
   for (int t = 0; t < 9; ++t) acc[t][0] = acc[t][1] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const int ntask = B * nstrips * nchunk;
-  for (int task = blockIdx.x * 4 + wave; task < ntask; task += gridDim.x * 4) {
-    const int x0 = (task % nstrips) * kWgPx;
-    const int y0 = ((task / nstrips) % nchunk) * rows;
-    const int b = task / (nstrips * nchunk);
-    int ny, nx;
-    extent_of(ext, b, H, W, ny, nx);
-    const int y1 = min(y0 + rows, ny);
-    if (x0 >= nx || y0 >= y1) continue;
+  StripShare<kWgPx, kWgRows> share(ext, B, H, W, chunks, wid, nw);
+  while (share.more()) {
+    const auto [b, x0, y0, y1, ny, nx] = share.next();
+    if (y0 >= y1) continue;
     const uint32_t img = (uint32_t)b * H * rowbytes;
     // dz: 16 B of a row per lane, pixel lane / 4 of 16; X: pixel x0 - 1 + lane.
     // X's addresses are clamped into the extent, its values masked when split.
@@ -535,7 +533,7 @@ conv_in_wgrad_kernel(const float* __restrict__ f0, const float* __restrict__ f1,
       sm.sums[wave][t][4 + g][cb * 16 + n] = a[3];
     }
   __syncthreads();
-  float* P = partials + (int64_t)blockIdx.x * kInOut;
+  float* P = partials + (int64_t)blk * kInOut;
   constexpr int kPer = (kInOut + 255) / 256;
   float prev[kPer];  // (all loads before the first store)
 #pragma unroll
@@ -556,21 +554,15 @@ conv_in_wgrad_kernel(const float* __restrict__ f0, const float* __restrict__ f1,
   }
 }
 
-// Equal shares of the strips' rows for all waves, in multiples of the four
-// steps of the loop; at most 32 rows in a batch of uneven entries, whose
-// padding is skipped.
-inline int strip_rows(const int32_t* ext, int B, int H, int nstrips, int nblocks) {
-  const int64_t waves = 4 * (int64_t)nblocks;
-  int64_t rows = ((int64_t)B * nstrips * H + waves - 1) / waves;
-  rows = (rows + 3) / 4 * 4;
-  return (int)(ext && rows > 32 ? 32 : rows);
+// (a start of the march: three rows of operands before the first products)
+inline int wgrad_chunks(const int32_t* ext, int B, int H, int W, int nblocks) {
+  return strip_chunks(ext, B, H, W, kWgPx, kWgRows, 3, 4 * nblocks);
 }
 
 int wgrad3x3_launch(const void* act, const void* dz, const int32_t* ext, int B, int H, int W, int nblocks,
                     float* partials, int accumulate, hipStream_t st) {
-  const int nstrips = (W + kWgPx - 1) / kWgPx, rows = strip_rows(ext, B, H, nstrips, nblocks);
   hipLaunchKernelGGL(wgrad3x3_kernel, dim3(nblocks), dim3(256), 0, st, (const bf16*)act, (const bf16*)dz, ext, B, H, W,
-                     nstrips, (H + rows - 1) / rows, rows, accumulate, partials);
+                     wgrad_chunks(ext, B, H, W, nblocks), accumulate, partials);
   IGM_CHECK_LAUNCH();
   return 0;
 }
@@ -586,14 +578,13 @@ extern "C" int igm_conv3x3_bwd_bf16(const void* act, const void* dz, const void*
   IGM_CHECK_ARG(nblocks >= 1 && B >= 1 && H >= 1 && W >= 1, "bad sizes");
   const int64_t bytes = (int64_t)B * H * W * kC * 2;
   IGM_CHECK_ARG(bytes < (int64_t)kOOB, "activations above 2 GiB (32-bit buffer offsets)");
-  const int nstrips = (W + kWgPx - 1) / kWgPx, rows = strip_rows(extents, B, H, nstrips, nblocks);
-  const int acc = accumulate ? 1 : 0, nchunk = (H + rows - 1) / rows;
+  const int acc = accumulate ? 1 : 0, chunks = wgrad_chunks(extents, B, H, W, nblocks);
   hipStream_t st = (hipStream_t)stream;
   switch (conv_store_mode(bytes, true)) {
 #define IGM_STORE_CASE(ST)                                                                                          \
   case ST:                                                                                                          \
     hipLaunchKernelGGL((bwd3x3_kernel<ST>), dim3(nblocks), dim3(256), 0, st, (const bf16*)act,              \
-                       (const bf16*)dz, (const bf16*)wpacked_dgrad, extents, B, H, W, nstrips, nchunk, rows, acc,   \
+                       (const bf16*)dz, (const bf16*)wpacked_dgrad, extents, B, H, W, chunks, acc,                  \
                        (bf16*)dz_below, partials);                                                                  \
     break;
     IGM_STORE_CASE(kStoreCached)
@@ -613,10 +604,9 @@ extern "C" int igm_conv_in_wgrad_partials(const float* f0, const float* f1, cons
   IGM_CHECK_ARG(f0 && f1 && f2 && f3 && f4 && dz1 && partials, "null pointer");
   IGM_CHECK_ARG(nblocks >= 1 && B >= 1 && H >= 1 && W >= 1, "bad sizes");
   IGM_CHECK_ARG((int64_t)B * H * W * kC * 2 < (int64_t)kOOB, "activations above 2 GiB (32-bit buffer offsets)");
-  const int nstrips = (W + kWgPx - 1) / kWgPx, rows = strip_rows(extents, B, H, nstrips, nblocks);
   hipLaunchKernelGGL(conv_in_wgrad_kernel, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, f0, f1, f2, f3, f4, fb, fr,
-                     fc, (const bf16*)dz1, extents, B, H, W, nstrips, (H + rows - 1) / rows, rows, accumulate ? 1 : 0,
-                     partials);
+                     fc, (const bf16*)dz1, extents, B, H, W, wgrad_chunks(extents, B, H, W, nblocks),
+                     accumulate ? 1 : 0, partials);
   IGM_CHECK_LAUNCH();
   return 0;
 }
