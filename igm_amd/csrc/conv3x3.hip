@@ -17,11 +17,13 @@
 // rate of a plain copy of such buffers (23 to 25 us; 5.7 TB/s), where the
 // products alone take 7.5 us.  The earlier kernel, which staged tiles of rows
 // in LDS between barriers, took 33 us.  Two layers in one launch move half
-// the bytes and are bound by instruction issue: a product takes 8 of its 16
-// matrix cycles of the SIMD's issue and the other instructions 4 each, about
-// 150 of them per 72 products.  37 to 42 us for both at 1000 x 1000, 8.5 at
-// 100 x 100 (5.1 for one).
+// the bytes and are bound by the matrix and the vector instructions of the one
+// wave a SIMD holds, 72 products of 16 cycles and about 170 others of 4 per row
+// and layer, which hardly overlap: 39 us for both at 1000 x 1000, 31 of them in
+// the waves (43 % of the time in products), 8.5 at 100 x 100 (5.1 for one).
 #include "conv_common.hpp"
+
+#include <type_traits>
 
 namespace igm {
 
@@ -303,6 +305,14 @@ __device__ __forceinline__ u32x4 px_right(u32x4 v) {
 // The second layer is complete on 62 of the 64 columns, and a wave computes
 // two more rows of the first layer than it owns.  Outside the extent the
 // first layer is zero, the second one's padding.
+//
+// The row that a layer has finished gets its bias, LeakyReLU and rounding while
+// the other layer multiplies: its second layer's rows during the first layer's
+// next one, the first layer's row during the second layer's first six taps,
+// which don't read it, three vector instructions after each product.  Left to
+// the scheduler, a layer's chains ran one after the other with waits between:
+// an emulator pass at 1000 x 1000 385 us, now 363; 1500 x 1500 88 us a launch,
+// now 83.
 template <int ST>
 __global__ void __launch_bounds__(256, 1)
 conv3x3_pair_kernel(const ConvArgs a) {
@@ -344,78 +354,137 @@ conv3x3_pair_kernel(const ConvArgs a) {
 #pragma unroll
     for (int f = 0; f < 6; ++f) r[f] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff[f], so, 0);
   };
+  f32x4 bl_r[2][2];
+  bf16x8 wr[2][18];
+#pragma unroll
+  for (int l = 0; l < 2; ++l)
+#pragma unroll
+    for (int f = 0; f < 18; ++f) wr[l][f] = as_bf16x8(wl[l][f][t.lane]);
+#pragma unroll
+  for (int l = 0; l < 2; ++l)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) bl_r[l][c] = *reinterpret_cast<const f32x4*>(&bl[l][8 * t.g + 4 * c]);
   u32x4 r[3][6];  // input rows
   u32x4 m[3][6];  // the first layer's rows
 #pragma unroll
   for (int i = 0; i < 3; ++i) load_row(r[i], t.y0 - 2 + i);
 
-  // row y of layer l from its input rows; `between` runs after row ra's last use
-  auto layer = [&](int l, int y, const u32x4 (&ra)[6], const u32x4 (&rb)[6], const u32x4 (&rc)[6],
-                   u32x4 (&o)[4], auto&& between) {
-    f32x4 acc[4][2];
-#pragma unroll
-    for (int tap = 0; tap < 9; ++tap) {
-      const u32x4 (&rr)[6] = tap < 3 ? ra : (tap < 6 ? rb : rc);
-      const bf16x8 w0 = as_bf16x8(wl[l][2 * tap][t.lane]), w1 = as_bf16x8(wl[l][2 * tap + 1][t.lane]);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const bf16x8 v = as_bf16x8(rr[q + tap % 3]);
-        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-        acc[q][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0, v, tap == 0 ? zero : acc[q][0], 0, 0, 0);
-        acc[q][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1, v, tap == 0 ? zero : acc[q][1], 0, 0, 0);
-      }
-      if (tap == 2) between();
-    }
-    const bool rv = (y >= 0) & (y < t.ny);
-    const f32x4 b01[2] = {*reinterpret_cast<const f32x4*>(&bl[l][8 * t.g]),
-                          *reinterpret_cast<const f32x4*>(&bl[l][8 * t.g + 4])};
+  // The products of one tap of layer l.
+  auto mult = [&](int l, int tap, f32x4 (&acc)[4][2], const u32x4 (&ra)[6], const u32x4 (&rb)[6], const u32x4 (&rc)[6]) __attribute__((always_inline)) {
+    const u32x4 (&rr)[6] = tap < 3 ? ra : (tap < 6 ? rb : rc);
+    const bf16x8 w0 = wr[l][2 * tap], w1 = wr[l][2 * tap + 1];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      bf16x8 h;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        float v = acc[q][e >> 2][e & 3] + b01[e >> 2][e & 3];
-        v = fmaxf(v, 0.01f * v);
-        h[e] = f2bf(v);
-      }
-      o[q] = __builtin_bit_cast(u32x4, h);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o[q][i] = (xin[q] & rv) ? o[q][i] : 0u;
+      const bf16x8 v = as_bf16x8(rr[q + tap % 3]);
+      const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+      acc[q][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0, v, tap == 0 ? zero : acc[q][0], 0, 0, 0);
+      acc[q][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1, v, tap == 0 ? zero : acc[q][1], 0, 0, 0);
     }
   };
-  // row c of the first layer, from r[I], r[I + 1], r[I + 2], into m[I]
-  auto first = [&](int I, int c) {
-    u32x4 o[4];
-    layer(0, c, r[I], r[(I + 1) % 3], r[(I + 2) % 3], o, [&] { load_row(r[I], c + 2); });
+  // Part u of 8 of a row's epilogue: half of slot group u / 2's channels.
+  auto finish = [&](int l, int u, const f32x4 (&acc)[4][2], bool rv, u32x4 (&o)[4]) __attribute__((always_inline)) {
+    const int q = u >> 1, c = u & 1;
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    bf16x4 h;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) m[I][q + 1] = o[q];
-    m[I][0] = px_left(o[3]);
-    m[I][5] = px_right(o[0]);
+    for (int e = 0; e < 4; ++e) {
+      float v = acc[q][c][e] + bl_r[l][c][e];
+      v = fmaxf(v, 0.01f * v);
+      h[e] = f2bf(v);
+    }
+    const uint2 w = __builtin_bit_cast(uint2, h);
+    const bool ok = xin[q] & rv;
+    o[q][2 * c] = ok ? w.x : 0u;
+    o[q][2 * c + 1] = ok ? w.y : 0u;
   };
-  // row y of the output: the first layer's row y + 1, then the second layer
-  auto step = [&](int I, int y) {
-    first(I, y + 1);
-    u32x4 o[4];
-    layer(1, y, m[(I + 1) % 3], m[(I + 2) % 3], m[I], o, [] {});
+  // a row of the first layer, with its neighbours' end pixels
+  auto put = [&](u32x4 (&d)[6], const u32x4 (&o)[4]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) store_px<ST>(o[q], rout, ooff[q], t.img + (uint32_t)y * t.rowbytes);
+    for (int q = 0; q < 4; ++q) d[q + 1] = o[q];
+    d[0] = px_left(o[3]);
+    d[5] = px_right(o[0]);
   };
-  first(0, t.y0 - 1);
-  first(1, t.y0);
-  // whole groups of three rows as one block of instructions (the scheduler
-  // overlaps a layer's epilogue with the next one's products), then the rest
+  // One tap's products with `valu` vector instructions between each two.
+  auto interleave = [](auto valu) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, valu.value, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  f32x4 acc0[4][2], acc1[4][2];
+  // Row c of the first layer, from r[I], r[I + 1], r[I + 2], and between its
+  // products the epilogue of the second layer's row c - 2, or (HEAD) of the
+  // first layer's row c - 1, into m[I - 1].
+  auto first = [&](int I, int c, auto head) __attribute__((always_inline)) {
+    u32x4 o[4];
+    const uint32_t so = t.img + (uint32_t)(c - 2) * t.rowbytes;
+    const bool rv = (c - 1 >= 0) & (c - 1 < t.ny);
+#pragma unroll
+    for (int tap = 0; tap < 9; ++tap) {
+      mult(0, tap, acc0, r[I], r[(I + 1) % 3], r[(I + 2) % 3]);
+      if (tap < 8) finish(head.value ? 0 : 1, tap, acc1, head.value ? rv : true, o);
+      if (tap == 3) load_row(r[I], c + 2);
+      if (!head.value && tap >= 2 && tap % 2 == 0) store_px<ST>(o[tap / 2 - 1], rout, ooff[tap / 2 - 1], so);
+      if (head.value && tap == 8) put(m[(I + 2) % 3], o);
+      interleave(std::integral_constant<int, 3>{});
+    }
+  };
+  // row y of the second layer: its products, and the epilogue of the first
+  // layer's row y + 1, into m[I], which the last three taps read
+  auto second = [&](int I, int y) __attribute__((always_inline)) {
+    const bool rv = y + 1 < t.ny;
+    u32x4 o[4];
+#pragma unroll
+    for (int tap = 0; tap < 9; ++tap) {
+      mult(1, tap, acc1, m[(I + 1) % 3], m[(I + 2) % 3], m[I]);
+      if (tap < 2) finish(0, 2 * tap, acc0, rv, o), finish(0, 2 * tap + 1, acc0, rv, o);
+      else if (tap < 6) finish(0, tap + 2, acc0, rv, o);
+      if (tap == 5) put(m[I], o);
+      if (tap < 2) interleave(std::integral_constant<int, 5>{});
+      else interleave(std::integral_constant<int, 3>{});
+    }
+  };
+  auto step = [&](int I, int y) __attribute__((always_inline)) {
+    first(I, y + 1, std::false_type{});
+    second(I, y);
+  };
+  // the first layer's rows y0 - 1, y0 and y0 + 1
+#pragma unroll
+  for (int tap = 0; tap < 9; ++tap) mult(0, tap, acc0, r[0], r[1], r[2]);
+  load_row(r[0], t.y0 + 1);
+  {
+    u32x4 o[4];
+    const bool rv = t.y0 > 0;
+#pragma unroll
+    for (int tap = 0; tap < 9; ++tap) {
+      mult(0, tap, acc1, r[1], r[2], r[0]);
+      if (tap < 8) finish(0, tap, acc0, rv, o);
+      if (tap == 3) load_row(r[1], t.y0 + 2);
+      if (tap == 8) put(m[0], o);
+      interleave(std::integral_constant<int, 3>{});
+    }
+  }
   int y = t.y0;
-  for (; y + 3 <= yv; y += 3) {
-    step(2, y);
-    step(0, y + 1);
-    step(1, y + 2);
+  first(2, y + 1, std::true_type{});
+  second(2, y);
+  for (++y; y + 3 <= yv; y += 3) {
+    step(0, y);
+    step(1, y + 1);
+    step(2, y + 2);
   }
   if (yv - y == 1) {
-    step(2, y);
+    step(0, y);
   } else if (yv - y == 2) {
-    step(2, y);
-    step(0, y + 1);
+    step(0, y);
+    step(1, y + 1);
   }
+  u32x4 o[4];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) finish(1, u, acc1, true, o);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) store_px<ST>(o[q], rout, ooff[q], t.img + (uint32_t)(yv - 1) * t.rowbytes);
 }
 
 }  // namespace igm
