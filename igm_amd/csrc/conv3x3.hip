@@ -19,8 +19,10 @@
 // in LDS between barriers, took 33 us.  Two layers in one launch move half
 // the bytes and are bound by the matrix and the vector instructions of the one
 // wave a SIMD holds, 72 products of 16 cycles and about 170 others of 4 per row
-// and layer, which hardly overlap: 39 us for both at 1000 x 1000, 31 of them in
-// the waves (43 % of the time in products), 8.5 at 100 x 100 (5.1 for one).
+// and layer, which hardly overlap (43 % of a wave's time are products): 30 us
+// for both at 1000 x 1000, where one layer from and to the last-level cache
+// takes 18.6, and 7.3 at 100 x 100 (4.7 for one), most of it the launch and the
+// first loads.
 #include "conv_common.hpp"
 
 #include <type_traits>
@@ -108,6 +110,26 @@ __device__ __forceinline__ ConvTile conv_tile(const ConvArgs& a, int own) {
 __device__ __forceinline__ const u32x4* weight_frag(const bf16* wt, const ConvTile& t, int tap, int cb) {
   return conv_weight_frag(wt, t.n, t.g, tap, cb);
 }
+// A block's weights on their way to LDS.  Their loads, and then the first rows',
+// are under way together before a wave waits for the former: one latency at the
+// start of a launch instead of two.  Two layers at 100 x 100 8.3 -> 7.3 us, 256 x
+// 319 10.8 -> 9.3, 1000 x 1000 35 -> 30; one layer 5.15 -> 4.7, 6.2 -> 5.65 and
+// 19.6 -> 18.6.
+template <int F, int N>  // F fragments, at least 4 N - 3
+__device__ __forceinline__ void weights_load(u32x4 (&w)[N], const bf16* const (&wt)[2], const ConvTile& t) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int f = min(4 * i + (int)(threadIdx.x >> 6), F - 1);
+    const int l = f >= 18 ? 1 : 0, k = f - 18 * l;
+    w[i] = *conv_weight_frag(wt[l], t.n, t.g, k >> 1, k & 1);
+  }
+}
+template <int N>
+__device__ __forceinline__ void weights_put(u32x4 (*wl)[64], const u32x4 (&w)[N]) {
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < N; ++i) wl[4 * i + (threadIdx.x >> 6)][threadIdx.x & 63] = w[i];
+}
 // A row's 16 B per lane to byte offset off (kOOB: dropped) of the row at so.
 // The row's offset is added to the lane's, not given in the instruction's
 // scalar offset: behind a 16-B store without one the compiler keeps the wait
@@ -138,13 +160,30 @@ __device__ __forceinline__ uint32_t px_off(const ConvTile& t, int x, bool ok) {
 template <int MODE, int ST, bool HEAD>
 __global__ void __launch_bounds__(256, 2)
 conv3x3_kernel(const ConvArgs a) {
-  __shared__ u32x4 wl[18][64];
+  __shared__ u32x4 wl[20][64];  // 18 fragments (and two unused)
   const ConvTile t = conv_tile(a, kStripPx);
-  for (int f = threadIdx.x >> 6; f < 18; f += 4) wl[f][t.lane] = *weight_frag(a.wt[0], t, f >> 1, f & 1);
+  u32x4 ws[5];
+  weights_load<18>(ws, a.wt, t);
+  const int xl = t.x0 + 8 * (t.n >> 1) + (t.n & 1);  // pixel of slot q: xl + 2 q
+  const int yv = t.x0 < t.nx ? min(t.y1, t.ny) : t.y0;  // rows y0 .. yv - 1 are computed
+  // fragment f: pixels xl + f - 1, f = 0 .. 8
+  uint32_t voff[9];
+#pragma unroll
+  for (int f = 0; f < 9; ++f) voff[f] = px_off(t, xl + f - 1, (xl + f - 1 >= 0) & (xl + f - 1 < t.nx));
+  auto load_row = [&](u32x4 (&r)[9], int y) {
+    const bool ok = (y >= 0) & (y < t.ny) & (y <= yv);
+    const rsrc_t rs = make_rsrc(a.in, ok ? t.bytes : 0u);
+    const uint32_t so = ok ? t.img + (uint32_t)y * t.rowbytes : 0u;
+#pragma unroll
+    for (int f = 0; f < 9; ++f) r[f] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff[f], so, 0);
+  };
+  u32x4 r0[9], r1[9], r2[9];
+  load_row(r0, t.y0 - 1);
+  load_row(r1, t.y0);
+  load_row(r2, t.y0 + 1);
+  weights_put(wl, ws);
   __syncthreads();
   if (!t.live) return;
-
-  const int xl = t.x0 + 8 * (t.n >> 1) + (t.n & 1);  // pixel of slot q: xl + 2 q
   uint32_t ooff[4];
   bool xin[4];
 #pragma unroll
@@ -169,7 +208,6 @@ conv3x3_kernel(const ConvArgs a) {
         __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[e]), ry, co + e < a.cout ? o + 4 * e : kOOB, 0, 0);
     }
   };
-  const int yv = t.x0 < t.nx ? min(t.y1, t.ny) : t.y0;  // rows y0 .. yv - 1 are computed
   for (int y = max(yv, t.y0); y < t.y1; ++y) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -200,18 +238,6 @@ conv3x3_kernel(const ConvArgs a) {
       }
     }
   }
-  // fragment f: pixels xl + f - 1, f = 0 .. 8
-  uint32_t voff[9];
-#pragma unroll
-  for (int f = 0; f < 9; ++f) voff[f] = px_off(t, xl + f - 1, (xl + f - 1 >= 0) & (xl + f - 1 < t.nx));
-  auto load_row = [&](u32x4 (&r)[9], int y) {
-    const bool ok = (y >= 0) & (y < t.ny) & (y <= yv);
-    const rsrc_t rs = make_rsrc(a.in, ok ? t.bytes : 0u);
-    const uint32_t so = ok ? t.img + (uint32_t)y * t.rowbytes : 0u;
-#pragma unroll
-    for (int f = 0; f < 9; ++f) r[f] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff[f], so, 0);
-  };
-
   // row y from input rows y - 1 (ra), y (rb), y + 1 (rc); loads row y + 2 into ra
   auto step = [&](int y, u32x4 (&ra)[9], const u32x4 (&rb)[9], const u32x4 (&rc)[9]) {
     const uint32_t so = t.img + (uint32_t)y * t.rowbytes;
@@ -270,10 +296,6 @@ conv3x3_kernel(const ConvArgs a) {
     }
   };
 
-  u32x4 r0[9], r1[9], r2[9];
-  load_row(r0, t.y0 - 1);
-  load_row(r1, t.y0);
-  load_row(r2, t.y0 + 1);
   for (int y = t.y0;; y += 3) {
     step(y, r0, r1, r2);
     if (y + 1 >= yv) break;
@@ -319,31 +341,11 @@ conv3x3_pair_kernel(const ConvArgs a) {
   __shared__ u32x4 wl[2][18][64];
   __shared__ __attribute__((aligned(16))) float bl[2][kC];
   const ConvTile t = conv_tile(a, kPairPx);
-#pragma unroll
-  for (int l = 0; l < 2; ++l) {
-    for (int f = threadIdx.x >> 6; f < 18; f += 4) wl[l][f][t.lane] = *weight_frag(a.wt[l], t, f >> 1, f & 1);
-    if (threadIdx.x < kC) bl[l][threadIdx.x] = a.bias[l][threadIdx.x];
-  }
-  __syncthreads();
-  if (!t.live) return;
+  u32x4 ws[9];
+  weights_load<36>(ws, a.wt, t);
+  const float bs = (threadIdx.x < kC ? a.bias[0] : a.bias[1])[threadIdx.x & (kC - 1)];
   const int xl = t.x0 - 1 + 4 * t.n;  // pixel of slot q: xl + q
-  uint32_t ooff[4];
-  bool xin[4];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int p = 4 * t.n + q;
-    ooff[q] = px_off(t, xl + q, (p >= 1) & (p <= kPairPx) & (xl + q < a.W));
-    xin[q] = (xl + q >= 0) & (xl + q < t.nx);
-  }
-  const rsrc_t rout = make_rsrc(a.out, t.bytes);
   const int yv = t.x0 < t.nx ? min(t.y1, t.ny) : t.y0;  // rows y0 .. yv - 1 are computed
-  for (int y = max(yv, t.y0); y < t.y1; ++y) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      store_px<kStoreCached>(u32x4{0, 0, 0, 0}, rout, ooff[q], t.img + y * t.rowbytes);
-  }
-  if (yv <= t.y0) return;
-
   uint32_t voff[6];  // fragment f: pixels xl + f - 1
 #pragma unroll
   for (int f = 0; f < 6; ++f) voff[f] = px_off(t, xl + f - 1, (xl + f - 1 >= 0) & (xl + f - 1 < t.nx));
@@ -354,6 +356,29 @@ conv3x3_pair_kernel(const ConvArgs a) {
 #pragma unroll
     for (int f = 0; f < 6; ++f) r[f] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff[f], so, 0);
   };
+  u32x4 r[3][6];  // input rows
+#pragma unroll
+  for (int i = 0; i < 3; ++i) load_row(r[i], t.y0 - 2 + i);
+  weights_put(&wl[0][0], ws);
+  if (threadIdx.x < 2 * kC) bl[threadIdx.x / kC][threadIdx.x & (kC - 1)] = bs;
+  __syncthreads();
+  if (!t.live) return;
+  uint32_t ooff[4];
+  bool xin[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int p = 4 * t.n + q;
+    ooff[q] = px_off(t, xl + q, (p >= 1) & (p <= kPairPx) & (xl + q < a.W));
+    xin[q] = (xl + q >= 0) & (xl + q < t.nx);
+  }
+  const rsrc_t rout = make_rsrc(a.out, t.bytes);
+  for (int y = max(yv, t.y0); y < t.y1; ++y) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      store_px<kStoreCached>(u32x4{0, 0, 0, 0}, rout, ooff[q], t.img + y * t.rowbytes);
+  }
+  if (yv <= t.y0) return;
+
   f32x4 bl_r[2][2];
   bf16x8 wr[2][18];
 #pragma unroll
@@ -364,10 +389,7 @@ conv3x3_pair_kernel(const ConvArgs a) {
   for (int l = 0; l < 2; ++l)
 #pragma unroll
     for (int c = 0; c < 2; ++c) bl_r[l][c] = *reinterpret_cast<const f32x4*>(&bl[l][8 * t.g + 4 * c]);
-  u32x4 r[3][6];  // input rows
   u32x4 m[3][6];  // the first layer's rows
-#pragma unroll
-  for (int i = 0; i < 3; ++i) load_row(r[i], t.y0 - 2 + i);
 
   // The products of one tap of layer l.
   auto mult = [&](int l, int tap, f32x4 (&acc)[4][2], const u32x4 (&ra)[6], const u32x4 (&rb)[6], const u32x4 (&rc)[6]) __attribute__((always_inline)) {
