@@ -188,7 +188,8 @@ wgrad3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const
 // 1 us a row and 8 us more.  Split by StripShare, 8 patches of 197 .. 294 cells
 // take 37 us and of 302 .. 394 cells 50 us; with equal blocks of rows of the
 // padded batch, dealt out in turn, 58 and 75.  At 410 .. 496 cells memory bounds
-// it again, and neighbouring strips out of step cost 6 us: 88, then 82.
+// it again, and neighbouring strips out of step cost 6 us: 88, where the padded
+// blocks took 82.
 template <int ST>
 __global__ void __launch_bounds__(256, 1)
 bwd3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const bf16* __restrict__ wt,
