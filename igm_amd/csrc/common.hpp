@@ -68,6 +68,20 @@ __device__ __forceinline__ rsrc_t make_rsrc(const void* p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, kRsrcWord3);
 }
 
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+// Every 16-B store goes through here: to byte offset off (kOOB: dropped), with
+// nothing in the instruction's scalar offset.  The store reads its data
+// registers after it has issued, and the compiler keeps the wait states until
+// they are written again only behind stores without a scalar offset.  (The ISA
+// documents exempt the other form, but a forward layer that used it, with two
+// waves on a SIMD, stored the next values in its last lanes.)  An offset of all
+// lanes is therefore added to off.
+template <int AUX = 0>
+__device__ __forceinline__ void store_b128(u32x4 v, rsrc_t r, uint32_t off) {
+  __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, AUX);
+}
+
 // MI355X dispatches the workgroups of a launch to its 8 XCDs round-robin
 // (workgroup p runs on XCD p % 8), and each XCD has an L2 of its own.
 // xcd_remap turns the dispatch index p of nb workgroups into a logical index

@@ -130,16 +130,6 @@ __device__ __forceinline__ void weights_put(u32x4 (*wl)[64], const u32x4 (&w)[N]
 #pragma unroll
   for (int i = 0; i < N; ++i) wl[4 * i + (threadIdx.x >> 6)][threadIdx.x & 63] = w[i];
 }
-// A row's 16 B per lane to byte offset off (kOOB: dropped) of the row at so.
-// The row's offset is added to the lane's, not given in the instruction's
-// scalar offset: behind a 16-B store without one the compiler keeps the wait
-// states that the store's data registers need before they are written again.
-// With one it adds none, and where two waves share a SIMD the last lanes'
-// data was then overwritten before it was read.
-template <int ST>
-__device__ __forceinline__ void store_px(u32x4 v, rsrc_t r, uint32_t off, uint32_t so) {
-  __builtin_amdgcn_raw_buffer_store_b128(v, r, off + so, 0, ST);
-}
 // byte offset of pixel x of a row, this lane's channels; kOOB unless ok
 __device__ __forceinline__ uint32_t px_off(const ConvTile& t, int x, bool ok) {
   return ok ? (uint32_t)(x * kC + 8 * t.g) * 2 : kOOB;
@@ -201,7 +191,7 @@ conv3x3_kernel(const ConvArgs a) {
     const int x = xl + 2 * q, co = 16 * c + 4 * t.g;
     const uint32_t o = ((x < a.W) & (co < a.cout)) ? (uint32_t)(x * a.cout + co) * 4 : kOOB;
     if (vec) {
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ry, o, 0, 0);
+      store_b128(__builtin_bit_cast(u32x4, v), ry, o);
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
@@ -211,7 +201,7 @@ conv3x3_kernel(const ConvArgs a) {
   for (int y = max(yv, t.y0); y < t.y1; ++y) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      store_px<kStoreCached>(u32x4{0, 0, 0, 0}, rout, ooff[q], t.img + y * t.rowbytes);
+      store_b128(u32x4{0, 0, 0, 0}, rout, ooff[q] + t.img + y * t.rowbytes);
       if constexpr (HEAD) {
 #pragma unroll
         for (int c = 0; c < 2; ++c) store_y(y, q, c, f32x4{0.f, 0.f, 0.f, 0.f});
@@ -282,7 +272,7 @@ conv3x3_kernel(const ConvArgs a) {
       u32x4 o = __builtin_bit_cast(u32x4, h);
 #pragma unroll
       for (int i = 0; i < 4; ++i) o[i] = xin[q] ? o[i] : 0u;
-      if (!HEAD || a.out) store_px<ST>(o, rout, ooff[q], so);
+      if (!HEAD || a.out) store_b128<ST>(o, rout, ooff[q] + so);
       if constexpr (HEAD) {
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
@@ -375,7 +365,7 @@ conv3x3_pair_kernel(const ConvArgs a) {
   for (int y = max(yv, t.y0); y < t.y1; ++y) {
 #pragma unroll
     for (int q = 0; q < 4; ++q)
-      store_px<kStoreCached>(u32x4{0, 0, 0, 0}, rout, ooff[q], t.img + y * t.rowbytes);
+      store_b128(u32x4{0, 0, 0, 0}, rout, ooff[q] + t.img + y * t.rowbytes);
   }
   if (yv <= t.y0) return;
 
@@ -448,7 +438,7 @@ conv3x3_pair_kernel(const ConvArgs a) {
       mult(0, tap, acc0, r[I], r[(I + 1) % 3], r[(I + 2) % 3]);
       if (tap < 8) finish(head.value ? 0 : 1, tap, acc1, head.value ? rv : true, o);
       if (tap == 3) load_row(r[I], c + 2);
-      if (!head.value && tap >= 2 && tap % 2 == 0) store_px<ST>(o[tap / 2 - 1], rout, ooff[tap / 2 - 1], so);
+      if (!head.value && tap >= 2 && tap % 2 == 0) store_b128<ST>(o[tap / 2 - 1], rout, ooff[tap / 2 - 1] + so);
       if (head.value && tap == 8) put(m[(I + 2) % 3], o);
       interleave(std::integral_constant<int, 3>{});
     }
@@ -506,7 +496,7 @@ conv3x3_pair_kernel(const ConvArgs a) {
 #pragma unroll
   for (int u = 0; u < 8; ++u) finish(1, u, acc1, true, o);
 #pragma unroll
-  for (int q = 0; q < 4; ++q) store_px<ST>(o[q], rout, ooff[q], t.img + (uint32_t)(yv - 1) * t.rowbytes);
+  for (int q = 0; q < 4; ++q) store_b128<ST>(o[q], rout, ooff[q] + t.img + (uint32_t)(yv - 1) * t.rowbytes);
 }
 
 }  // namespace igm

@@ -11,7 +11,6 @@ namespace igm {
 typedef __bf16 bf16;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kC = 32;   // hidden channels
 constexpr int kCin = 5;  // input fields

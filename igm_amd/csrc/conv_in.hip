@@ -152,7 +152,7 @@ conv_in_kernel(const float* __restrict__ f0, const float* __restrict__ f1, const
             const float a = acc[p][8 * c + e];
             v[e] = f2bf(__builtin_elementwise_maximum(a, 0.01f * a));  // LeakyReLU
           }
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ro, os[p] + 32 * c, 0, 0);
+          store_b128(__builtin_bit_cast(u32x4, v), ro, os[p] + 32 * c);
         }
       o += orow;
     }

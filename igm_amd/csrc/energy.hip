@@ -28,9 +28,6 @@
 
 namespace igm {
 
-// four dwords, the operand of the 16-byte buffer loads and stores
-typedef unsigned int v4u32 __attribute__((ext_vector_type(4)));
-
 namespace {
 thread_local std::string g_last_error;
 }
@@ -202,7 +199,7 @@ energy_pass_kernel(const PassArgs<T> a) {
         adam_step(m, g_u, g_v, a.omb1, a.omb2, a.alpha, a.eps, up[k], vp[k], un_, vn_);
         bstore(un_, make_rsrc(a.Uo, a.vel_bytes), on, k * kstep);
         bstore(vn_, make_rsrc(a.Vo, a.vel_bytes), on, k * kstep);
-        mstore(m, rM, om, k * mstep);
+        mstore(m, rM, om + k * mstep);
       };
       // output of node (jc, ic), level k (masked stores)
       auto emit = [&](int k, T g_u, T g_v) {
@@ -233,9 +230,9 @@ energy_pass_kernel(const PassArgs<T> a) {
         }
 #pragma unroll
         for (int i = 0; i < NZ / 2; ++i) {
-          const v4u32 x = {__float_as_uint(f[4 * i]), __float_as_uint(f[4 * i + 1]),
+          const u32x4 x = {__float_as_uint(f[4 * i]), __float_as_uint(f[4 * i + 1]),
                            __float_as_uint(f[4 * i + 2]), __float_as_uint(f[4 * i + 3])};
-          __builtin_amdgcn_raw_buffer_store_b128(x, rG, on, 16 * i, 0);
+          store_b128(x, rG, on + 16 * i);
         }
       }
 

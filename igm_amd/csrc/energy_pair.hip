@@ -231,7 +231,7 @@ energy_pair_kernel(const PassArgs<float> a) {
                   q_v[k]);
         if constexpr (M == kOneIter) {
           store_uv(q_u[k], q_v[k], o1, k);
-          mstore(m[k], rMo, om1, k * mstep);
+          mstore(m[k], rMo, om1 + k * mstep);
         } else {
           sm[sn][k][lane] = make_float4(m[k][0], m[k][1], m[k][2], m[k][3]);
           sq[sn][k][lane] = make_float2(q_u[k], q_v[k]);
@@ -245,7 +245,7 @@ energy_pair_kernel(const PassArgs<float> a) {
         T un_, vn_;
         adam_step(mk, g_u, g_v, a.omb1, a.omb2, alpha2, a.eps, p_u[k], p_v[k], un_, vn_);
         store_uv(un_, vn_, o2, k);
-        mstore(mk, rMo, om2, k * mstep);
+        mstore(mk, rMo, om2 + k * mstep);
       };
       auto stage_b_level = [&](LevelSweep<T, NZ>& sb, int k) {
         const float2 t = sq[sp][k][lane];

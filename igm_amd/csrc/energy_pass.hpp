@@ -66,23 +66,21 @@ __device__ __forceinline__ void mload(rsrc_t r, uint32_t voff, uint32_t soff, do
     m[2 * h + 1] = __hiloint2double((int)v[3], (int)v[2]);
   }
 }
-__device__ __forceinline__ void mstore(const float (&m)[4], rsrc_t r, uint32_t voff, uint32_t soff) {
-  typedef unsigned int u4 __attribute__((ext_vector_type(4)));
-  u4 v;
+__device__ __forceinline__ void mstore(const float (&m)[4], rsrc_t r, uint32_t off) {
+  u32x4 v;
 #pragma unroll
   for (int i = 0; i < 4; ++i) v[i] = __float_as_uint(m[i]);
-  __builtin_amdgcn_raw_buffer_store_b128(v, r, voff, soff, 0);
+  store_b128(v, r, off);
 }
-__device__ __forceinline__ void mstore(const double (&m)[4], rsrc_t r, uint32_t voff, uint32_t soff) {
-  typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void mstore(const double (&m)[4], rsrc_t r, uint32_t off) {
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    u4 v;
+    u32x4 v;
     v[0] = (unsigned)__double2loint(m[2 * h]);
     v[1] = (unsigned)__double2hiint(m[2 * h]);
     v[2] = (unsigned)__double2loint(m[2 * h + 1]);
     v[3] = (unsigned)__double2hiint(m[2 * h + 1]);
-    __builtin_amdgcn_raw_buffer_store_b128(v, r, voff + 16 * h, soff, 0);
+    store_b128(v, r, off + 16 * h);
   }
 }
 

@@ -131,7 +131,7 @@ energy_team_kernel(const PassArgs<float> a) {
         bstore(u, rUo, o, k * kstep);
         bstore(v, rVo, o, k * kstep);
       }
-      mstore(m, rMo, o == kOOB ? kOOB : 4u * o + k * mstep, 0);
+      mstore(m, rMo, (o == kOOB ? kOOB : 4u * o) + k * mstep);
     };
     const auto none = [](int, float, float) {};
 

@@ -229,8 +229,7 @@ bwd3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const b
       extent_of(ext, r / H, H, W, ny, nx);
       const int x0 = r % H < ny ? (max(nx, 0) + kWgPx - 1) / kWgPx * kWgPx : 0;
       for (int x = x0 + (lane >> 2); x < W; x += 16)
-        __builtin_amdgcn_raw_buffer_store_b128(u32x4{0, 0, 0, 0}, ro,
-                                               (uint32_t)r * rowbytes + (uint32_t)(x * kC * 2 + (lane & 3) * 16), 0, 0);
+        store_b128(u32x4{0, 0, 0, 0}, ro, (uint32_t)r * rowbytes + (uint32_t)(x * kC * 2 + (lane & 3) * 16));
     }
   }
   StripShare<kWgPx, kWgRows> share(ext, B, H, W, chunks, wid, nw);
@@ -334,7 +333,7 @@ bwd3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const b
         u32x4 v = __builtin_bit_cast(u32x4, h);
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] = xin[q] ? v[i] : 0u;
-        __builtin_amdgcn_raw_buffer_store_b128(v, ro, oo[q] + img + (uint32_t)(y + k) * rowbytes, 0, ST);
+        store_b128<ST>(v, ro, oo[q] + img + (uint32_t)(y + k) * rowbytes);
       }
     };
     // Two rows of both gradients in twelve slots.
