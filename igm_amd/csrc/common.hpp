@@ -129,9 +129,11 @@ __device__ __forceinline__ double scaled_pow(double x, double e, double d, doubl
 // rounding of e included): the float32 power y of the mantissa m, which is good
 // to 2^-22, and one third-order step of y (1 - r)^(-1/3), r = 1 - m y^3.  y^2 is
 // exact, the rounding of m y is put back into r, and the step and x^(e + 1/3)
-// are added with one rounding: 0.5 ulp at most, 0.29 in the root mean square
-// over [1e-10, 1e3] (pow: 0.7 and 0.30; two roundings and r as computed: 1.3 and
-// 0.42).  About 30 instructions where pow takes 250.
+// are added with one rounding.  The largest error sampled over [1e-10, 1e3] is
+// 0.50 ulp, 0.29 in the root mean square (pow: 0.7 and 0.30; two roundings and r
+// as computed: 1.3 and 0.42); over 3,100 values of all exponents, subnormal ones
+// too, x x^e as a pass computes it is within 1.61 x 2^-53.  About 30 instructions
+// where pow takes 250.
 __device__ __forceinline__ double pow_third(double x, double e) {
   const int ex = __builtin_amdgcn_frexp_exp(x), q = (int)floorf((float)ex * (1.0f / 3.0f) + 0.125f);
   const double m = __builtin_amdgcn_ldexp(__builtin_amdgcn_frexp_mant(x), ex - 3 * q);  // [1/2, 4)
