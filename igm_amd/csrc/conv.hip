@@ -378,8 +378,10 @@ wgrad1x1_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz,
   }
 }
 
-// Deterministic reduction of per-block partials P[nblk][stride], in two
-// stages.  Stage 1 (partials_group_sum_kernel): group g of R rows,
+// Deterministic reduction of one layer's per-block partials P[nblk][stride], in
+// two stages, for the calls that ask for one layer (igm_conv_wgrad_bf16,
+// igm_conv_in_wgrad, igm_conv_wgrad_reduce_f32); a network's layers go through
+// wgrad_reduce_layers_kernel.  Stage 1 (partials_group_sum_kernel): group g of R rows,
 // rows g*R .. min(nblk, (g+1)*R) - 1, is summed in row order into its first
 // row, in place; each (group, column) belongs to one thread, so the write
 // races with nothing, and the loads are issued 8 at a time.  Stage 2 sums
@@ -418,8 +420,8 @@ __device__ __forceinline__ int wgrad_kernel_pos(int taps, int src, int cout) {
   return co < cout ? (tap * kC + ci) * cout + co : -1;
 }
 
-// Stage 2 for a 3x3 or 1x1 layer: the group sums of entry src = ((tap * 32
-// + co) * 32 + ci) (then the 32 bias entries) scattered to dW (HWIO, cout
+// Stage 2 for a 3x3 or 1x1 layer: the group sums of each entry, in the order of
+// wgrad_kernel_pos (then the 32 bias entries), scattered to dW (HWIO, cout
 // output channels) and db.
 __global__ void __launch_bounds__(256)
 wgrad_reduce_kernel(const float* __restrict__ P, int ngroups, int R, int taps, int cout,
@@ -441,8 +443,9 @@ wgrad_reduce_kernel(const float* __restrict__ P, int ngroups, int R, int taps, i
 // The partial sums of every layer of a network into its flat gradient, in one
 // launch: a block takes 64 consecutive entries of one layer's rows, each of its
 // four waves every fourth row, in order, and wave 0 adds the four sums in order:
-// rows of zeros at the end, of blocks without work, change nothing.  Layer by layer in two stages these were 34 launches of 4 to 6 us
-// for 16 layers, which read 140 MB in all.
+// rows of zeros at the end, of blocks without work, change nothing.  Layer by
+// layer in two stages these were 34 launches of 4 to 6 us for 16 layers, which
+// read 140 MB in all.
 struct ReduceArgs {
   const float* part[3];  // layer 1, the 3x3 layers one after the other, the head
   int rows[3];
@@ -450,7 +453,6 @@ struct ReduceArgs {
   const int64_t* offs;   // kernel of layer l at g + offs[2 l], its bias at g + offs[2 l + 1]
   float* g;
 };
-constexpr int kWgIn = 9 * kCin * kC + kC, kWg9 = 9 * kC * kC + kC, kWg1 = kC * kC + kC;
 constexpr int reduce_blocks(int entries) { return (entries + 63) / 64; }
 __global__ void __launch_bounds__(256)
 wgrad_reduce_layers_kernel(const ReduceArgs a) {
@@ -502,8 +504,6 @@ inline void group_rows(int nblk, int* R, int* G) {
   *R = (nblk + *G - 1) / *G;
   *G = (nblk + *R - 1) / *R;
 }
-
-constexpr int kWgOut = 9 * kCin * kC + kC;  // floats of a block's partial sums of layer 1 (wgrad3x3.hip)
 
 // Stage 2 as a plain column sum: out[i] = sum over the group rows of P[.][i],
 // i < count
@@ -625,9 +625,9 @@ int igm_conv1x1_head_bwd(const float* dY, const void* a16, const float* w_hwio,
 }
 
 int64_t igm_wgrad_workspace_floats(int32_t taps, int32_t nblocks) {
-  if (taps == 9) return (int64_t)nblocks * (9 * 1024 + 32);
-  if (taps == 1) return (int64_t)nblocks * (1024 + 32);
-  if (taps == 0) return (int64_t)nblocks * (9 * 5 * 32 + 32);  // layer 1
+  if (taps == 9) return (int64_t)nblocks * kWg9;
+  if (taps == 1) return (int64_t)nblocks * kWg1;
+  if (taps == 0) return (int64_t)nblocks * kWgIn;  // layer 1
   return 0;
 }
 
@@ -660,7 +660,7 @@ int igm_conv_wgrad_reduce_f32(int32_t taps, int32_t cout, int32_t nblocks, float
   group_rows(nblocks, &R, &G);
   if (taps == 0) {
     // the layer-1 partial layout is [blk][1440 + 32] = [blk][n]: a plain column sum
-    const int n = kWgOut;
+    const int n = kWgIn;
     hipLaunchKernelGGL(partials_group_sum_kernel, dim3((n + 255) / 256, G), dim3(256), 0, st,
                        partials, nblocks, n, n, R);
     IGM_CHECK_LAUNCH();

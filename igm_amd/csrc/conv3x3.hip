@@ -107,9 +107,6 @@ __device__ __forceinline__ ConvTile conv_tile(const ConvArgs& a, int own) {
   t.img = (uint32_t)b * a.H * t.rowbytes;
   return t;
 }
-__device__ __forceinline__ const u32x4* weight_frag(const bf16* wt, const ConvTile& t, int tap, int cb) {
-  return conv_weight_frag(wt, t.n, t.g, tap, cb);
-}
 // A block's weights on their way to LDS.  Their loads, and then the first rows',
 // are under way together before a wave waits for the former: one latency at the
 // start of a launch instead of two.  Two layers at 100 x 100 8.3 -> 7.3 us, 256 x
@@ -137,7 +134,8 @@ __device__ __forceinline__ uint32_t px_off(const ConvTile& t, int x, bool ok) {
 
 // One layer.  MODE 0: out = LeakyReLU(conv + bias).  MODE 1 (dgrad): out =
 // conv * (aux > 0 ? 1 : 0.01), aux = activation of the layer below (its sign
-// is the sign of its pre-activation).  Slots n hold pairs of neighbouring
+// is the sign of its pre-activation); the network's backward pass runs
+// bwd3x3_kernel instead, this mode serves igm_conv3x3_dgrad_bf16.  Slots n hold pairs of neighbouring
 // pixels, 8 (n / 2) + 2 q + n % 2 for slot group q: an access of the wave
 // covers whole 128-B lines (interleaved by 4 n + q instead, half lines, 1500
 // x 1500 took 74 us a layer, now 60).  Tap column s of group q is then the

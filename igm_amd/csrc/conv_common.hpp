@@ -15,7 +15,10 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kC = 32;   // hidden channels
 constexpr int kCin = 5;  // input fields
 
-__device__ __forceinline__ float leaky(float x) { return x > 0.f ? x : 0.01f * x; }
+// floats of a block's partial sums of the weight gradient (kernel, then 32 of
+// the bias): layer 1, a 3x3 layer, the output layer
+constexpr int kWgIn = 9 * kCin * kC + kC, kWg9 = 9 * kC * kC + kC, kWg1 = kC * kC + kC;
+
 __device__ __forceinline__ float bf2f(bf16 h) { return (float)h; }
 __device__ __forceinline__ bf16 f2bf(float f) { return (bf16)f; }
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }

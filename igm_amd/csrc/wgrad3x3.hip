@@ -19,13 +19,15 @@
 // padded patches 40 us, with 256 blocks, one wave per SIMD (512: 1000 x 1000
 // 32.6 us).  The earlier kernel transposed with VALU packing into
 // block-wide LDS tiles, read by all waves between barriers: 39 and 62 us.
+//
+// wgrad3x3_kernel is the weight gradient alone and serves igm_conv_wgrad_bf16 and
+// igm_conv_wgrad_partials_bf16; the network's backward pass runs bwd3x3_kernel.
 #include "conv_common.hpp"
 
 namespace igm {
 
 constexpr int kWgPx = 32;                 // columns of a wave's strip: the K of one product
 constexpr int kWgRows = 4;                // rows of a round of the march
-constexpr int kWgEntries = 9 * kC * kC + kC;  // floats of a block's partial sums
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
@@ -45,7 +47,7 @@ __device__ __forceinline__ bf16x8 transposed(const bf16* s, int p, int cb) {
 // The sums of a block's four waves, in order, in the lanes' own layout: entry
 // ((tap * 4 + block) * 64 + lane) * 4 + e, then the bias.
 __device__ __forceinline__ void wave_sums(const f32x4 (&acc)[9][2][2], const f32x4 (&accb)[2],
-                                          f32x4 (&sums)[4][kWgEntries / 4], int blk, int accumulate, float* partials) {
+                                          f32x4 (&sums)[4][kWg9 / 4], int blk, int accumulate, float* partials) {
   const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4, wave = threadIdx.x >> 6;
   __syncthreads();
 #pragma unroll
@@ -57,19 +59,19 @@ __device__ __forceinline__ void wave_sums(const f32x4 (&acc)[9][2][2], const f32
     for (int c = 0; c < 2; ++c) sums[wave][9 * kC * kC / 4 + 4 * c + g] = accb[c];
   }
   __syncthreads();
-  f32x4* P = reinterpret_cast<f32x4*>(partials + (int64_t)blk * kWgEntries);
-  constexpr int kPer = (kWgEntries / 4 + 255) / 256;
+  f32x4* P = reinterpret_cast<f32x4*>(partials + (int64_t)blk * kWg9);
+  constexpr int kPer = (kWg9 / 4 + 255) / 256;
   f32x4 prev[kPer];
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
     const int q = threadIdx.x + 256 * k;
     prev[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (accumulate) prev[k] = P[q < kWgEntries / 4 ? q : 0];
+    if (accumulate) prev[k] = P[q < kWg9 / 4 ? q : 0];
   }
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
     const int q = threadIdx.x + 256 * k;
-    if (q < kWgEntries / 4) {
+    if (q < kWg9 / 4) {
       const f32x4 v = ((sums[0][q] + sums[1][q]) + sums[2][q]) + sums[3][q];
       P[q] = accumulate ? prev[k] + v : v;
     }
@@ -84,7 +86,7 @@ wgrad3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const
   constexpr int kStage = (kWgPx + 16 + kWgPx) * kC;
   __shared__ __attribute__((aligned(16))) union {
     bf16 rows[4][kStage];
-    f32x4 sums[4][kWgEntries / 4];
+    f32x4 sums[4][kWg9 / 4];
   } sm;
   const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -106,7 +108,8 @@ wgrad3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const
 
   StripShare<kWgPx, kWgRows> share(ext, B, H, W, chunks, wid, nw);
   while (share.more()) {
-    const auto [b, x0, y0, y1, ny, nx] = share.next();
+    const StripRange sr = share.next();
+    const int b = sr.b, x0 = sr.x0, y0 = sr.y0, y1 = sr.y1, ny = sr.ny, nx = sr.nx;
     if (y0 >= y1) continue;
     const uint32_t img = (uint32_t)b * H * rowbytes;
     // a lane's 16 B of a row: pixel lane / 4 of 16, chunk lane % 4
@@ -202,7 +205,7 @@ bwd3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const b
       bf16 act[4][4][kRowPx * kC], dz[4][4][kRowPx * kC];
       u32x4 w[18][64];
     } in;
-    f32x4 sums[4][kWgEntries / 4];
+    f32x4 sums[4][kWg9 / 4];
   } sm;
   const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -234,7 +237,8 @@ bwd3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const b
   }
   StripShare<kWgPx, kWgRows> share(ext, B, H, W, chunks, wid, nw);
   while (share.more()) {
-    const auto [b, x0, y0, y1, ny, nx] = share.next();
+    const StripRange sr = share.next();
+    const int b = sr.b, x0 = sr.x0, y0 = sr.y0, y1 = sr.y1, ny = sr.ny, nx = sr.nx;
     if (y0 >= y1) continue;
     const uint32_t img = (uint32_t)b * H * rowbytes;
     uint32_t oo[2];  // data gradient: pixel x0 + 16 q + n, channels 8 g .. 8 g + 7
@@ -417,8 +421,7 @@ bwd3x3_kernel(const bf16* __restrict__ act, const bf16* __restrict__ dz, const b
 // What bounds it: 1000 x 1000 takes 21 us (512 blocks, 23 with 256), 84 MB at
 // 4.0 TB/s; 8 x 496 x 496 padded patches 30 us.  Float32 FMAs from LDS tiles
 // took 90 and 168 us, with twice the rounding error.
-constexpr int kXc = 16;                        // channels of a split pixel
-constexpr int kInOut = 9 * kCin * kC + kC;     // floats of a block's partial sums
+constexpr int kXc = 16;  // channels of a split pixel
 
 __device__ __forceinline__ float split_sum(float h, float m, float l) {
   return __builtin_isfinite(h) ? (l + m) + h : h;
@@ -451,7 +454,8 @@ conv_in_wgrad_kernel(const float* __restrict__ f0, const float* __restrict__ f1,
 
   StripShare<kWgPx, kWgRows> share(ext, B, H, W, chunks, wid, nw);
   while (share.more()) {
-    const auto [b, x0, y0, y1, ny, nx] = share.next();
+    const StripRange sr = share.next();
+    const int b = sr.b, x0 = sr.x0, y0 = sr.y0, y1 = sr.y1, ny = sr.ny, nx = sr.nx;
     if (y0 >= y1) continue;
     const uint32_t img = (uint32_t)b * H * rowbytes;
     // dz: 16 B of a row per lane, pixel lane / 4 of 16; X: pixel x0 - 1 + lane.
@@ -543,18 +547,18 @@ conv_in_wgrad_kernel(const float* __restrict__ f0, const float* __restrict__ f1,
       sm.sums[wave][t][4 + g][cb * 16 + n] = a[3];
     }
   __syncthreads();
-  float* P = partials + (int64_t)blk * kInOut;
-  constexpr int kPer = (kInOut + 255) / 256;
+  float* P = partials + (int64_t)blk * kWgIn;
+  constexpr int kPer = (kWgIn + 255) / 256;
   float prev[kPer];  // (all loads before the first store)
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
     const int i = threadIdx.x + 256 * k;
-    prev[k] = (accumulate && i < kInOut) ? P[i] : 0.f;
+    prev[k] = (accumulate && i < kWgIn) ? P[i] : 0.f;
   }
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
     const int i = threadIdx.x + 256 * k;
-    if (i >= kInOut) continue;
+    if (i >= kWgIn) continue;
     const int co = i % kC, m = i / kC, t = m < 9 * kCin ? m / kCin : 4, ci = m < 9 * kCin ? m % kCin : 7;
     float v = 0.f;
 #pragma unroll
