@@ -13,15 +13,17 @@
 // operand.  Every output sums taps 0 .. 8 in order from zero and adds the
 // bias last, in all of these kernels: they agree bit for bit.
 //
-// What bounds them: at 1000 x 1000 one layer moves 128 MB in 22.6 us, the
-// rate of a plain copy of such buffers (23 to 25 us; 5.7 TB/s), where the
-// products alone take 7.5 us.  The earlier kernel, which staged tiles of rows
-// in LDS between barriers, took 33 us.  Two layers in one launch move half
-// the bytes and are bound by the matrix and the vector instructions of the one
-// wave a SIMD holds, 72 products of 16 cycles and about 170 others of 4 per row
-// and layer, which hardly overlap (43 % of a wave's time are products): 30 us
-// for both at 1000 x 1000, where one layer from and to the last-level cache
-// takes 18.6, and 7.3 at 100 x 100 (4.7 for one), most of it the launch and the
+// What bounds them: one layer, memory.  At 1000 x 1000 it moves 128 MB, where
+// the products alone take 7.5 us: 18.2 us back and forth between two buffers,
+// which the last-level cache holds, and 29.5 us (4.3 TB/s) in a pass that keeps
+// its activations, sixteen buffers from and to HBM.  (From one buffer to
+// another over and over, as the benchmark times it, 21 us; the earlier kernel,
+// which staged tiles of rows in LDS between barriers, 33.)  Two layers in one
+// launch move half the bytes and are bound by the matrix and the vector
+// instructions of the one wave a SIMD holds, 72 products of 16 cycles and about
+// 170 others of 4 per row and layer, which hardly overlap (43 % of a wave's time
+// are products): at 1000 x 1000 31 us for both in a loop and 33.6 in a pass, at
+// 100 x 100 7.1 either way (4.5 and 5.1 for one), most of it the launch and the
 // first loads.
 #include "conv_common.hpp"
 
@@ -109,9 +111,9 @@ __device__ __forceinline__ ConvTile conv_tile(const ConvArgs& a, int own) {
 }
 // A block's weights on their way to LDS.  Their loads, and then the first rows',
 // are under way together before a wave waits for the former: one latency at the
-// start of a launch instead of two.  Two layers at 100 x 100 8.3 -> 7.3 us, 256 x
-// 319 10.8 -> 9.3, 1000 x 1000 35 -> 30; one layer 5.15 -> 4.7, 6.2 -> 5.65 and
-// 19.6 -> 18.6.
+// start of a launch instead of two.  In a loop between two buffers, two layers at
+// 100 x 100 8.3 -> 7.3 us, 256 x 319 10.8 -> 9.3, 1000 x 1000 35 -> 30; one layer
+// 5.15 -> 4.7, 6.2 -> 5.65 and 19.6 -> 18.6.
 template <int F, int N>  // F fragments, at least 4 N - 3
 __device__ __forceinline__ void weights_load(u32x4 (&w)[N], const bf16* const (&wt)[2], const ConvTile& t) {
 #pragma unroll

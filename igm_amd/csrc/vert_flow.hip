@@ -13,9 +13,9 @@
 // of its four neighbours; the neighbours' values come through L1/L2, so HBM
 // sees U, V, thk, topg about once (88 B/cell in, 40 B/cell of W out at Nz 10).
 // For that the rows of the grid are dealt to the XCDs in bands: with row after
-// row on another XCD every L2 fetched its neighbours' rows too, and 1000 x 1000
-// at Nz 10 took 30 us, now 22 (136 MB, 6.2 TB/s; 500 x 500 10.5 and 8.4, Nz 20
-// 56 and 41).
+// row on another XCD every L2 fetched its neighbours' rows too, and the kernel
+// took 30 us at 1000 x 1000, Nz 10, now 22 (136 MB, 6.2 TB/s; 500 x 500 10.5 and
+// 8.4, Nz 20 56 and 41).  (Calls of the process, bound by the host: 36 and 35.)
 #include "common.hpp"
 #include "../../include/igm_amd.h"
 

@@ -40,7 +40,10 @@ def glorot_uniform(shape, gen):
 
 class Partials:
     """Partial sums of the weight gradients: layer 1's, the 3x3 layers' and the
-    output layer's, with their rows, in one buffer (16-B aligned parts)."""
+    output layer's, with their rows, in one buffer (16-B aligned parts).  All
+    layers' at once, for one reduction launch: with 256 rows of 37 KB per 3x3
+    layer 147 MB for 16 layers, where a buffer that every layer's own reduction
+    used in turn was 19 MB."""
 
     def __init__(self, rows, n3x3, device):
         lib = L.load()
