@@ -5,7 +5,14 @@ of test_gpu_pair, whose grids are the teams'.
 
 Which kernel a grid takes is read from the workspace: 6 doubles per block of
 the two-iteration pass, more than 3 per block of the one-iteration pass on
-these grids; the teams would be fewer blocks."""
+these grids; the teams would be fewer blocks.
+
+IGM_PAIR_WAVES, which a process reads once, keeps small grids on the march too:
+a child process with it set takes the grids of test_gpu_pair through it."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -13,6 +20,7 @@ import torch
 from igm_amd import _lib as L
 from igm_amd.solver import LegacyAdamState, solve
 from tests.helpers import small_glacier
+from tests.test_gpu_pair import CASES as SMALL
 from tests.test_gpu_pair import first_mismatch, gpu_op
 from tests.test_gpu_pair import test_pair_equals_two_single_passes as check_pair
 from tests.test_gpu_pair import test_pair_interleaved_layouts as check_layouts
@@ -60,3 +68,26 @@ def test_solve_on_the_march(dev, nz, nit, patience, delta):
     assert first_mismatch(r2.U, r1.U) is None and first_mismatch(r2.V, r1.V) is None
     c1, c2 = np.asarray(r1.costs), np.asarray(r2.costs)
     assert c1.shape == c2.shape and np.all(np.abs(c2 - c1) <= 1e-12 * np.abs(c1))
+
+
+SMALL_GRIDS = """
+import torch
+from igm_amd import _lib as L
+from tests import test_gpu_march as M
+dev = torch.device("cuda:0")
+# 100 x 100: 2 strips of 100 row blocks, 50 blocks; the teams take 200
+assert L.load().igm_energy_workspace_doubles(1, 100, 100) == 6 * 50
+for ny, nx, nz in M.SMALL:
+    M.check_pair(dev, ny, nx, nz)
+for ny, nx, nz in ((100, 100, 10), (37, 131, 5), (5, 7, 4), (61, 60, 12)):
+    M.check_layouts(dev, ny, nx, nz)
+    M.check_fresh(dev, ny, nx, nz)
+"""
+
+
+def test_small_grids_on_the_march(dev):
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    path = os.pathsep.join(p for p in (root, os.environ.get("PYTHONPATH")) if p)
+    r = subprocess.run([sys.executable, "-c", SMALL_GRIDS], cwd=root, timeout=100, capture_output=True, text=True,
+                       env=dict(os.environ, IGM_PAIR_WAVES="1024", PYTHONPATH=path))
+    assert r.returncode == 0, r.stdout[-1000:] + r.stderr[-3000:]
